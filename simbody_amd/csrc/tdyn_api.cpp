@@ -81,6 +81,63 @@ void pack_body_params(const tdyn_tree_desc& d, int b, double* P) {
     if (d.mobilizer[b-1] == TDYN_BUSHING) P[PRM_EULER] = 2.0;   // runs as a Free body with x-y-z angles, u = qdot
 }
 
+void pack_joint_consts(const tdyn_tree_desc& d, int b, double* C) {
+    for (int k = 0; k < PRM_STRIDE; ++k) C[k] = 0.0;
+    using LD = long double;
+    const double *RB = d.X_BM + 12*(b-1), *pB = RB + 9, *RF = d.X_PF + 12*(b-1), *pF = RF + 9;
+    const int p = d.parent[b-1];
+    // the parent's M frame (Ground's is Ground): R_MF = R_PM^T R_PF, l = R_PM^T (p_PF - p_PM)
+    static const double I12[12] = {1, 0, 0, 0, 1, 0, 0, 0, 1, 0, 0, 0};
+    const double* XP = p == 0 ? I12 : d.X_BM + 12*(p-1);
+    for (int r = 0; r < 3; ++r) {
+        LD l = 0;
+        for (int k = 0; k < 3; ++k) l += (LD)XP[3*k + r] * ((LD)pF[k] - (LD)XP[9 + k]);
+        C[JC_L + r] = (double)l;
+        for (int c = 0; c < 3; ++c) {
+            LD x = 0;
+            for (int k = 0; k < 3; ++k) x += (LD)XP[3*k + r] * (LD)RF[3*k + c];
+            C[JC_R + 3*r + c] = (double)x;
+        }
+    }
+    // mass properties about M's origin: v = com - p_BM in B, then to M axes
+    const LD m = d.mass[b-1];
+    LD cB[3], v[3], cc = 0, vv = 0;
+    for (int k = 0; k < 3; ++k) {
+        cB[k] = d.com_B[3*(b-1) + k]; v[k] = cB[k] - (LD)pB[k];
+        cc += cB[k]*cB[k]; vv += v[k]*v[k];
+    }
+    const double* I6 = d.inertia_B + 6*(b-1);
+    LD I[3][3], T[3][3];
+    for (int r = 0; r < 3; ++r)
+        for (int c = 0; c < 3; ++c) {
+            const LD x = r == c ? I6[r] : I6[r + c == 1 ? 3 : r + c == 2 ? 4 : 5];
+            I[r][c] = x - m*((r == c ? cc : (LD)0) - cB[r]*cB[c]) + m*((r == c ? vv : (LD)0) - v[r]*v[c]);
+        }
+    for (int r = 0; r < 3; ++r)
+        for (int c = 0; c < 3; ++c) {
+            T[r][c] = 0;
+            for (int k = 0; k < 3; ++k) T[r][c] += (LD)RB[3*k + r] * I[k][c];
+        }
+    static const int rr[6] = {0, 1, 2, 0, 0, 1}, rc[6] = {0, 1, 2, 1, 2, 2};
+    for (int e = 0; e < 6; ++e) {
+        LD x = 0;
+        for (int k = 0; k < 3; ++k) x += T[rr[e]][k] * (LD)RB[3*k + rc[e]];
+        C[JC_I + e] = (double)x;
+    }
+    C[JC_M] = d.mass[b-1];
+    for (int r = 0; r < 3; ++r) {
+        LD c = 0, o = 0;
+        for (int k = 0; k < 3; ++k) { c += (LD)RB[3*k + r] * v[k]; o -= (LD)RB[3*k + r] * (LD)pB[k]; }
+        C[JC_C + r] = (double)(m*c); C[JC_B + r] = (double)o;
+        for (int k = 0; k < 3; ++k) C[JC_RB + 3*r + k] = RB[3*k + r];
+    }
+}
+bool identity_joints(const double* C, int nb) {
+    for (int b = 0; b < nb; ++b)
+        for (int k = 0; k < 9; ++k) if (C[b*PRM_STRIDE + JC_R + k] != (k % 4 == 0 ? 1.0 : 0.0)) return false;
+    return true;
+}
+
 bool any_reversed(const tdyn_tree_desc& d) {
     if (!d.reversed) return false;
     for (int b = 0; b < d.nb; ++b) if (d.reversed[b]) return true;
@@ -237,7 +294,9 @@ int ensure_rollout_buffers(tdyn_batch* b, int precision) {
     if (b->vec.p && b->ny_max == ny) return TDYN_OK;
     b->ny_max = 0;
     // 8 extra rows: the chain evaluator prefetches fixed-size q/u windows
-    if ((e = b->vec.alloc((size_t)11 * ny * L + 8 * L)) != hipSuccess ||
+    size_t nvec = (size_t)11 * ny * L + 8 * L;
+    if (b->is_chain && tdyn_batch::joint_tiles((int)L, ny)) nvec = std::max(nvec, (size_t)11 * ny * ((L + 63) / 64 * 64));
+    if ((e = b->vec.alloc(nvec)) != hipSuccess ||
         (e = b->uscale.alloc((size_t)std::max(1, b->max_nu) * L)) != hipSuccess ||
         (e = b->t.alloc(L)) != hipSuccess || (e = b->h.alloc(L)) != hipSuccess ||
         (e = b->t_end.alloc(L)) != hipSuccess || (e = b->status.alloc(L)) != hipSuccess ||
@@ -389,6 +448,18 @@ int tdyn_batch_create(const tdyn_tree_desc* trees, int n_trees, const int32_t* t
     B->stream_stride = tdyn::tstream::scratch_doubles(B->dmax, B->max_nb);
     B->group_stride = tdyn::tgroup::scratch_doubles(B->max_nb);
     B->idf = B->is_chain && identity_frames(trees[0]);
+    std::vector<double> prm_j; std::vector<int4> body_j;
+    if (B->is_chain) {
+        const int nb = trees[0].nb;
+        prm_j.resize((size_t)nb * PRM_STRIDE);
+        for (int b = 1; b <= nb; ++b) {
+            const int ty = trees[0].mobilizer[b-1];
+            pack_joint_consts(trees[0], b, prm_j.data() + (size_t)(b-1) * PRM_STRIDE);
+            body_j.push_back(make_int4(ty, B->g_rows, B->tc_rows, 0));
+            B->g_rows += jt_g(ty); B->tc_rows += jt_tc(ty);
+        }
+        B->jidf = identity_joints(prm_j.data(), nb);
+    }
     {
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) == hipSuccess &&
@@ -428,6 +499,8 @@ int tdyn_batch_create(const tdyn_tree_desc* trees, int n_trees, const int32_t* t
         (e = B->body_b.upload(body_b)) != hipSuccess ||
         (e = B->child_idx.upload(child_idx.empty() ? std::vector<int>{0} : child_idx)) != hipSuccess ||
         (e = B->prm.upload(prm)) != hipSuccess ||
+        (e = B->prm_j.upload(prm_j)) != hipSuccess ||
+        (e = B->body_j.upload(body_j)) != hipSuccess ||
         (e = B->tree_a.upload(B->h_tree_a)) != hipSuccess ||
         (e = B->tree_b.upload(B->h_tree_b)) != hipSuccess ||
         (e = B->gravity.upload(grav)) != hipSuccess ||

@@ -1,13 +1,12 @@
-// Chain-evaluator rollout kernels: one model per lane, FP64.
-#include "tdyn_rkm_chain.hpp"
+// Chain rollout kernels in joint frames: one model per lane (serving slots,
+// whose number is a multiple of 64), FP64.
+#include "tdyn_rkm_joint.hpp"
 
 namespace tdyn {
 
 hipError_t launch_chain_fp64_lane(const RkmArgs& a, hipStream_t s, bool f0_only) {
-    // the derivative alone (f0_only) is the general form's bit for bit, so
-    // identity frames need no separate build there
-    if (a.idf && !f0_only) return launch_chain_t<chain::IdF<chain::PrmL>, double>(a, s, false);
-    return launch_chain_t<chain::PrmL, double>(a, s, f0_only);
+    return a.jidf ? launch_joint_i<joint::PrmT, true, true>(a, s, f0_only)
+                  : launch_joint_i<joint::PrmT, false, true>(a, s, f0_only);
 }
 
 } // namespace tdyn

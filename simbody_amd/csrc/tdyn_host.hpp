@@ -38,6 +38,11 @@ template <class T> struct DBuf {
 // The PRM_STRIDE model constants of body b (1-based) of tree d: X_PF, X_MB =
 // X_BM^-1, mass, mass center, unit inertia G = I/m about Bo, p_BM.
 void pack_body_params(const tdyn_tree_desc& d, int b, double* P);
+// The JC_* constants of body b (1-based) of tree d (tdyn_joint.hpp), formed in
+// extended precision and rounded once.
+void pack_joint_consts(const tdyn_tree_desc& d, int b, double* C);
+// True when all nb bodies' R_MF of such constants are the identity.
+bool identity_joints(const double* C, int nb);
 // True when every body's X_PF is the identity and X_BM has no rotation.
 bool identity_frames(const tdyn_tree_desc& d);
 // True when some body's mobilizer is reversed.
@@ -81,6 +86,9 @@ struct tdyn_batch {
     tdyn::host::DBuf<int> inst;          // instance of each lane
     bool permuted = false;               // lanes are not in instance order
     tdyn::host::DBuf<double> prm, gravity, scratch, prm_bfs;
+    tdyn::host::DBuf<double> prm_j; tdyn::host::DBuf<int4> body_j;   // joint-frame tables (chains)
+    bool jidf = false;           // every R_MF is the identity
+    int g_rows = 0, tc_rows = 0; // G and trig rows per lane of the joint-frame kernels
     tdyn::host::DBuf<int> op_status;     // per instance: status of the last operator that formed D
     // rollout state
     tdyn::host::DBuf<double> vec, uscale, t, h, t_end;
@@ -125,9 +133,15 @@ struct tdyn_batch {
     int plan_waves = 0;
     RkmCfg cfg{};
 
+    // Whether the joint-frame kernels keep the rollout state of n chains in
+    // blocks of 64 lanes: always from 64 instances, and below while the block's
+    // unused lanes cost little (64 MiB).
+    static bool joint_tiles(int n, int ny) { return n >= 64 || (size_t)tdyn::NVEC * ny * 64 * sizeof(double) <= ((size_t)64 << 20); }
+
     DevTables tables() const {
         DevTables T;
         T.body_a = body_a.p; T.body_b = body_b.p; T.child_idx = child_idx.p; T.prm = prm.p;
+        T.prm_j = prm_j.p; T.body_j = body_j.p;
         T.tree_a = tree_a.p; T.tree_b = tree_b.p; T.gravity = gravity.p; T.pre = pre.p; T.bfs = bfs.p; T.lvl = lvl.p;
         T.bfs_b = bfs_b.p; T.prm_bfs = prm_bfs.p;
         T.cons_t = any_cons ? cons_t.p : nullptr; T.cons_a = cons_a.p; T.cons_p = cons_p.p;
@@ -139,7 +153,7 @@ struct tdyn_batch {
         std::memset(&a, 0, sizeof(a));
         a.T = tables(); a.tree_of = uniform ? nullptr : tree_of.p; a.n_inst = n_inst; a.L = n_inst;
         a.scratch = scratch.p; a.rec_stride = max_rec + 24; a.off = {q_off.p, u_off.p, b_off.p}; a.inst = permuted ? inst.p : nullptr;
-        a.status = op_status.p;
+        a.status = op_status.p; a.jidf = jidf ? 1 : 0;
         a.cons_ws = any_cons ? cons_ws.p : nullptr;
         return a;
     }
@@ -159,6 +173,8 @@ struct tdyn_batch {
         a.presc = roll_known_p; a.udot_known = roll_known_u;
         if (roll_motion) { a.motion = roll_motion; a.presc = motion_flags.p; a.udot_known = motion_udot.p; }
         a.idf = (a.chain ? idf : idf_all) ? 1 : 0;
+        a.jidf = jidf ? 1 : 0; a.g_rows = g_rows; a.tc_rows = tc_rows;
+        a.tile = a.chain && precision == 0 && joint_tiles(n_inst, ny_max) ? 1 : 0;
         a.ext = (any_rev || any_euler || any_bendstretch || any_bushing || a.presc) ? 1 : 0;
         a.vec_aos = rollout_aos ? 1 : 0;
         a.stream_dmax = dmax;

@@ -59,6 +59,17 @@ enum {
                        angles and p_FM, u = qdot, H_FM the Gimbal's angle columns) */, PRM_STRIDE = 40
 };
 
+// Per-body constants of the joint-frame recursion (tdyn_joint.hpp), PRM_STRIDE
+// doubles per body: R_MF, the rotation from F to the parent's M axes; F's
+// origin in the parent's M frame; mass; mass times the mass center, and the
+// inertia about M's origin (xx yy zz xy xz yz), M axes; the body origin in M;
+// R_MB, the rotation from B to M axes.  (Ground's M frame is Ground.)
+enum { JC_R = 0, JC_L = 9, JC_M = 12, JC_C = 13, JC_I = 16, JC_B = 22, JC_RB = 25 };
+// Hand-over values of one body between the joint-frame sweeps: the entries of
+// G that are not known beforehand with DI*eps, and the trig values of q.
+__host__ __device__ constexpr int jt_g(int t) { return t == UNIVERSAL ? 10 : t == BALL ? 12 : 6; }
+__host__ __device__ constexpr int jt_tc(int t) { return t == PIN ? 2 : t == SLIDER ? 0 : t == UNIVERSAL ? 4 : 1; }
+
 // Per-body record in the per-lane scratch (doubles, relative to rec_off).
 // Stored structure-of-arrays across lanes: scratch[(rec_off + k) * L + lane].
 enum {
@@ -93,6 +104,8 @@ struct DevTables {
     const int4* body_b;      // per global body: child_begin, child_count, rec_off, -
     const int* child_idx;    // local body numbers
     const double* prm;       // PRM_STRIDE per global body
+    const double* prm_j;     // the same bodies' JC_* constants (batches of one chain)
+    const int4* body_j;      // per global body: mobilizer, first G row, first trig row, -
     const int4* tree_a;      // per tree: nb, nq, nu, body_off
     const int4* tree_b;      // per tree: rec_size, nquat, hand-over base of the chain evaluator, lvl offset
     const double* gravity;   // per tree: 4 doubles
@@ -159,6 +172,7 @@ struct OpArgs {
     DevTables T;
     const int* tree_of;      // null: every instance uses tree 0
     int n_inst;
+    int jidf;                // as in RkmArgs
     int L;                   // lane pitch of the scratch
     double* scratch;
     int rec_stride;          // doubles of scratch per lane (per-lane record layout of mixed-tree batches)
@@ -208,6 +222,11 @@ struct RkmArgs {
     RkmCfg cfg;
     int precision;           // 0 = FP64, 1 = mixed, 2/3 = FP64 with single-precision G (and trig) rows
     int chain;               // 1: uniform serial-chain model, use the register-resident chain evaluator
+    int jidf;                // joint-frame kernels: every R_MF is the identity
+    int g_rows, tc_rows;     // their G and trig rows per lane (body_j)
+    int tile;                // 1: vec in blocks of 64 lanes, row k of vector v of lane l at
+                             // ((l/64 * NVEC + v) * ny_max + k) * 64 + l%64 (and prm_lane in such blocks
+                             // of nb*PRM_STRIDE + 3 rows): the joint-frame kernels
     int idf;                 // chain evaluator: every frame is an identity rotation at the joints
                              // (R_PF = I, p_PF = 0, R_MB = I), so the frame products are skipped
     int ext;                 // some body's mobilizer is reversed (PRM_REV), uses Euler angles (PRM_EULER)
@@ -283,13 +302,15 @@ __host__ __device__ inline int blocks(int n) { return (n + BW - 1) / BW; }
 __host__ __device__ inline int scratch_doubles(int nbmax) { return NF * BW * blocks(nbmax); }
 __host__ __device__ inline int at(int j) { return (j / BW) * NF * BW + j % BW; }
 } // namespace tgroup
-// Entry k of state vector v of a lane, in either layout.
-__device__ __forceinline__ double& vec_at(const RkmArgs& a, int v, int lane, int k) {
-    return a.vec_aos ? a.vec[((size_t)v * a.L + lane) * a.ny_max + k] : a.vec[((size_t)v * a.ny_max + k) * a.L + lane];
-}
 // Rollout state vectors (rows of ny_max * L doubles in RkmArgs::vec): y, y0,
 // f0, fa, fb, ysave, y1, ystage, yerr and the mixed path's Kahan rows.
 enum { VY = 0, VY0 = 1, VF0 = 2, VFA = 3, VFB = 4, VYS = 5, VY1 = 6, VYT = 7, VYE = 8, VC0 = 9, VC1 = 10, NVEC = 11 };
+
+// Entry k of state vector v of a lane, in any layout.
+__device__ __forceinline__ double& vec_at(const RkmArgs& a, int v, int lane, int k) {
+    if (a.tile) return a.vec[(((size_t)(lane >> 6) * NVEC + v) * a.ny_max + k) * 64 + (lane & 63)];
+    return a.vec_aos ? a.vec[((size_t)v * a.L + lane) * a.ny_max + k] : a.vec[((size_t)v * a.ny_max + k) * a.L + lane];
+}
 
 hipError_t launch_rkm_init(const RkmArgs& a, double t0, hipStream_t s);
 // The initial projection of the lanes whose trees carry constraints

@@ -2481,8 +2481,9 @@ __global__ void __launch_bounds__(64) k_srv_admit(RkmArgs a, const double* rec, 
     const int np = nb * PRM_STRIDE + 3;
     const size_t L = a.L;
     double* prm_lane = const_cast<double*>(a.prm_lane);
-    for (int k = threadIdx.x; k < np; k += blockDim.x) prm_lane[(size_t)k * L + slot] = r[k];
-    for (int k = threadIdx.x; k < nq + nu; k += blockDim.x) a.vec[(size_t)k * L + slot] = r[np + k];   // VY
+    for (int k = threadIdx.x; k < np; k += blockDim.x)
+        prm_lane[a.tile ? ((size_t)(slot >> 6) * np + k) * 64 + (slot & 63) : (size_t)k * L + slot] = r[k];
+    for (int k = threadIdx.x; k < nq + nu; k += blockDim.x) vec_at(a, VY, slot, k) = r[np + k];
     double* fa = const_cast<double*>(a.fapp) + 6 * (size_t)a.off.b_off[slot];
     for (int k = threadIdx.x; k < 6 * (nb + 1); k += blockDim.x) fa[k] = r[np + nq + nu + 1 + k];
     __syncthreads();
@@ -2501,7 +2502,7 @@ __global__ void k_srv_collect(RkmArgs a, const int* slots, int n, double* out, i
     const int ny = ta.y + ta.z;
     const size_t L = a.L;
     double* o = out + (size_t)i * out_stride;
-    for (int k = 0; k < ny; ++k) o[k] = a.vec[(size_t)k * L + slot];
+    for (int k = 0; k < ny; ++k) o[k] = vec_at(a, VY, slot, k);
     o[ny] = a.t[slot];
     outi[5*i] = a.status[slot];
     for (int k = 0; k < 4; ++k) outi[5*i + 1 + k] = a.stats[4*slot + k];

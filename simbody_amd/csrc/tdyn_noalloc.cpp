@@ -122,6 +122,10 @@ extern "C" int tdyn_rollout_noalloc(tdyn_batch* b, double* q, double* u, const d
     a.scratch = reinterpret_cast<double*>(base + o_rec);
     a.vec = reinterpret_cast<double*>(base + o_vec);
     a.ny_max = ny;
+    // chains in joint frames: their blocks of 64 lanes where these fit in the
+    // records' and vectors' room, else rows of one pitch
+    a.tile = a.chain && sizeof(double) * (size_t)NVEC * ny * ((L + 63) / 64 * 64) <= o_us ? 1 : 0;
+    if (a.tile) a.vec = reinterpret_cast<double*>(base);
     a.uscale = reinterpret_cast<double*>(base + o_us);
     a.t = reinterpret_cast<double*>(base + o_t);
     a.h = reinterpret_cast<double*>(base + o_h);

@@ -39,13 +39,14 @@ struct tdyn_server {
     std::vector<int> free_list;
     std::vector<char> occupied;
     bool idf = false;      // every model admitted so far has identity joint frames
+    bool jidf = true;      // and identity rotations between its joints
     ~tdyn_server() { if (B) tdyn_batch_destroy(B); }
     int rec_stride() const { return nb * PRM_STRIDE + 3 + nq + nu + 1 + 6 * (nb + 1); }
     RkmArgs rk() const {
         RkmArgs a = B->rk();
         a.chain = 1;
         a.prm_lane = prm_lane.p;
-        a.idf = idf ? 1 : 0;
+        a.idf = idf ? 1 : 0; a.jidf = jidf ? 1 : 0;
         return a;
     }
 };
@@ -168,7 +169,12 @@ int tdyn_server_admit(tdyn_server* sv, int n, const tdyn_tree_desc* trees, const
     for (int i = 0; i < k; ++i) {
         double* r = sv->rec_host.p + (size_t)i * stride;
         const tdyn_tree_desc& d = trees[i];
-        for (int b = 1; b <= nb; ++b) pack_body_params(d, b, r + (size_t)(b-1) * PRM_STRIDE);
+        // the FP64 slots run in joint frames, the mixed ones in Ground
+        for (int b = 1; b <= nb; ++b) {
+            double* c = r + (size_t)(b-1) * PRM_STRIDE;
+            if (sv->B->precision == 0) pack_joint_consts(d, b, c); else pack_body_params(d, b, c);
+        }
+        if (sv->B->precision == 0) sv->jidf = sv->jidf && identity_joints(r, nb);
         double* x = r + (size_t)nb * PRM_STRIDE;
         x[0] = d.gravity[0]; x[1] = d.gravity[1]; x[2] = d.gravity[2];
         x += 3;
