@@ -110,6 +110,60 @@ TDJ void shift_mass(art& P, const d3& r) {
     P.J = {{-b0.x, -b1.y, -b2.z, -b1.x, -b2.x, -b2.y}};
 }
 
+// The same after a Pin about z (row z of F and of J zero), after a Universal
+// (row x zero; J is j e e^T and F is e f^T with e normal to x).
+TDJ void shift_pin(art& P, const d3& r) {
+    const d3 c0 = cross(r, d3{P.M.a[0], P.M.a[3], P.M.a[4]}), c1 = cross(r, d3{P.M.a[3], P.M.a[1], P.M.a[5]}),
+             c2 = cross(r, d3{P.M.a[4], P.M.a[5], P.M.a[2]});
+    const d3 a0 = cross(r, row(P.F, 0)), a1 = cross(r, row(P.F, 1));
+    P.F[0] += c0.x; P.F[1] += c1.x; P.F[2] += c2.x;
+    P.F[3] += c0.y; P.F[4] += c1.y; P.F[5] += c2.y;
+    P.F[6] = c0.z; P.F[7] = c1.z; P.F[8] = c2.z;
+    const d3 b0 = cross(row(P.F, 0), r), b1 = cross(row(P.F, 1), r), b2 = cross(row(P.F, 2), r);
+    P.J.a[0] += a0.x - b0.x; P.J.a[1] += a1.y - b1.y; P.J.a[2] = -b2.z;
+    P.J.a[3] += a0.y - b1.x; P.J.a[4] = a0.z - b2.x; P.J.a[5] = a1.z - b2.y;
+}
+TDJ void shift_universal(art& P, const d3& r) {
+    const d3 c0 = cross(r, d3{P.M.a[0], P.M.a[3], P.M.a[4]}), c1 = cross(r, d3{P.M.a[3], P.M.a[1], P.M.a[5]}),
+             c2 = cross(r, d3{P.M.a[4], P.M.a[5], P.M.a[2]});
+    const d3 a1 = cross(r, row(P.F, 1)), a2 = cross(r, row(P.F, 2));
+    P.F[0] = c0.x; P.F[1] = c1.x; P.F[2] = c2.x;
+    P.F[3] += c0.y; P.F[4] += c1.y; P.F[5] += c2.y;
+    P.F[6] += c0.z; P.F[7] += c1.z; P.F[8] += c2.z;
+    const d3 b0 = cross(row(P.F, 0), r), b1 = cross(row(P.F, 1), r), b2 = cross(row(P.F, 2), r);
+    P.J.a[0] = -b0.x; P.J.a[1] += a1.y - b1.y; P.J.a[2] += a2.z - b2.z;
+    P.J.a[3] = -b1.x; P.J.a[4] = -b2.x; P.J.a[5] += a1.z - b2.y;
+}
+
+// sin and cos for |x| < 2^20, the library's beyond.  x - k pi/2 in three parts
+// (Cody and Waite; the first is exact in one fused multiply-add), then
+// polynomials in r^2 through the Chebyshev nodes of [0, (pi/4)^2] (largest
+// error 2e-17) and the rest of r to first order: 40 instructions where the
+// library's small-argument path takes 130, under 1 ulp as that is.  One angle
+// per body and derivative made it a sixth of a chain derivative.
+TDJ void sincos_joint(double x, double* sp, double* cp) {
+    if (!(fabs(x) < 1048576.0)) { sincos(x, sp, cp); return; }
+    const double k = rint(x * 0.6366197723675814);
+    const double t = fma(-k, 1.5707963267948966, x);
+    const double r = fma(-k, 6.123233995736766e-17, t);
+    const double lo = fma(-k, -1.4973849048591698e-33, fma(-k, 6.123233995736766e-17, t - r));
+    const double z = r*r;
+    const double ps = fma(z, fma(z, fma(z, fma(z, fma(z, 1.591810123027412e-10, -2.5051131455427946e-08),
+                                                2.755731610068303e-06), -0.0001984126983675497),
+                                 0.008333333333330946), -0.16666666666666666);
+    const double pc = fma(z, fma(z, fma(z, fma(z, fma(z, -1.1382614868556325e-11, 2.0876146024689747e-09),
+                                                -2.7557317270560326e-07), 2.4801587298763433e-05),
+                                 -0.0013888888888887395), 0.041666666666666664);
+    const double hz = 0.5*z;
+    const double sn = r + fma(r*z, ps, fma(-hz, lo, lo));
+    const double w = 1.0 - hz;
+    const double cs = w + (((1.0 - w) - hz) + fma(z*z, pc, -(r*lo)));
+    const int n = (int)k;
+    const double a = (n & 1) ? cs : sn, b = (n & 1) ? sn : cs;
+    *sp = (n & 2) ? -a : a;
+    *cp = ((n + 1) & 2) ? -b : b;
+}
+
 // ---------------------------------------------------------------------------
 // Joints.  J axes: where the hinge columns are unit vectors.  Pin: the body's
 // M axes; Slider: the same (= F axes); Universal: F turned by the first angle;
@@ -129,8 +183,8 @@ template <int T> struct Jnt {
     d3 p;                       // Slider, Free: p_FM
     // trig / normalization values of q
     static TDJ void trig(const double* q, double* tc) {
-        if constexpr (T == PIN) sincos(q[0], &tc[1], &tc[0]);
-        else if constexpr (T == UNIVERSAL) { sincos(q[0], &tc[1], &tc[0]); sincos(q[1], &tc[3], &tc[2]); }
+        if constexpr (T == PIN) sincos_joint(q[0], &tc[1], &tc[0]);
+        else if constexpr (T == UNIVERSAL) { sincos_joint(q[0], &tc[1], &tc[0]); sincos_joint(q[1], &tc[3], &tc[2]); }
         else if constexpr (Dim<T>::quat) tc[0] = 1.0 / sqrt(q[0]*q[0] + q[1]*q[1] + q[2]*q[2] + q[3]*q[3]);
     }
     TDJ void set(const double* q, const double* tc) {
@@ -308,21 +362,23 @@ TDJ bool solve6(const art& P, const double* b, double* x) {
 
 // ---------------------------------------------------------------------------
 // Elimination of one joint, J axes.  In: P and z of the body with its
-// children, tau the applied mobility forces along the hinge columns.  Out: G
+// children, tau the applied mobility forces along the hinge columns (TAU).  Out: G
 // (Dim::G values without the known ones) and DI*eps into g[], and P, z become
 // P+ and z + G eps (the bias P+ ab is added by the caller).  Returns whether D
 // was not positive definite.
 // ---------------------------------------------------------------------------
-template <int T> TDJ bool eliminate(art& P, wf& z, const double* tau, double* g) {
+template <int T, bool TAU> TDJ bool eliminate(art& P, wf& z, const double* tau, double* g) {
     double* F = P.F;
+    auto ta = [&](int k) { return TAU ? tau[k] : 0.0; };
+    auto ep = [&](int k, double z) { return TAU ? tau[k] - z : -z; };
     if constexpr (T == PIN) {
         const double D = P.J.a[2], o = 1.0 / D;
         const double ux = P.J.a[4], uy = P.J.a[5];
         const d3 uv = row(F, 2);
         const double gx = ux*o, gy = uy*o;
         const d3 gv = {uv.x*o, uv.y*o, uv.z*o};
-        const double eps = tau[0] - z.w.z;
-        z.w.x += gx*eps; z.w.y += gy*eps; z.w.z = tau[0];
+        const double eps = ep(0, z.w.z);
+        z.w.x += gx*eps; z.w.y += gy*eps; z.w.z = ta(0);
         z.v = z.v + eps*gv;
         P.J.a[0] -= gx*ux; P.J.a[1] -= gy*uy; P.J.a[3] -= gx*uy;
         P.J.a[2] = 0; P.J.a[4] = 0; P.J.a[5] = 0;
@@ -341,9 +397,9 @@ template <int T> TDJ bool eliminate(art& P, wf& z, const double* tau, double* g)
         const double uy = P.M.a[3], uz = P.M.a[4];
         const d3 ga = {ua.x*o, ua.y*o, ua.z*o};
         const double gy = uy*o, gz = uz*o;
-        const double eps = tau[0] - z.v.x;
+        const double eps = ep(0, z.v.x);
         z.w = z.w + eps*ga;
-        z.v.x = tau[0]; z.v.y += gy*eps; z.v.z += gz*eps;
+        z.v.x = ta(0); z.v.y += gy*eps; z.v.z += gz*eps;
         P.J.a[0] -= ga.x*ua.x; P.J.a[1] -= ga.y*ua.y; P.J.a[2] -= ga.z*ua.z;
         P.J.a[3] -= ga.x*ua.y; P.J.a[4] -= ga.x*ua.z; P.J.a[5] -= ga.y*ua.z;
         F[0] = 0; F[3] = 0; F[6] = 0;
@@ -362,8 +418,8 @@ template <int T> TDJ bool eliminate(art& P, wf& z, const double* tau, double* g)
         const double gzx = ax*i00 + ay*i01, gzy = ax*i01 + ay*i11;
         const d3 gx = {fx.x*i00 + fy.x*i01, fx.y*i00 + fy.y*i01, fx.z*i00 + fy.z*i01};
         const d3 gy = {fx.x*i01 + fy.x*i11, fx.y*i01 + fy.y*i11, fx.z*i01 + fy.z*i11};
-        const double e0 = tau[0] - z.w.x, e1 = tau[1] - z.w.y;
-        z.w.x = tau[0]; z.w.y = tau[1]; z.w.z += gzx*e0 + gzy*e1;
+        const double e0 = ep(0, z.w.x), e1 = ep(1, z.w.y);
+        z.w.x = ta(0); z.w.y = ta(1); z.w.z += gzx*e0 + gzy*e1;
         z.v.x += gx.x*e0 + gy.x*e1; z.v.y += gx.y*e0 + gy.y*e1; z.v.z += gx.z*e0 + gy.z*e1;
         P.J.a[2] -= gzx*ax + gzy*ay;
         P.J.a[0] = 0; P.J.a[1] = 0; P.J.a[3] = 0; P.J.a[4] = 0; P.J.a[5] = 0;
@@ -388,8 +444,8 @@ template <int T> TDJ bool eliminate(art& P, wf& z, const double* tau, double* g)
             G[3*l+1] = F[l]*i01 + F[3+l]*i11 + F[6+l]*i12;
             G[3*l+2] = F[l]*i02 + F[3+l]*i12 + F[6+l]*i22;
         }
-        const d3 e = d3{tau[0], tau[1], tau[2]} - z.w;
-        z.w = {tau[0], tau[1], tau[2]};
+        const d3 e = {ep(0, z.w.x), ep(1, z.w.y), ep(2, z.w.z)};
+        z.w = {ta(0), ta(1), ta(2)};
         z.v = z.v + mulF(G, e);
 #pragma unroll
         for (int l = 0; l < 3; ++l)
@@ -406,10 +462,9 @@ template <int T> TDJ bool eliminate(art& P, wf& z, const double* tau, double* g)
         return !(det > 0.0);
     } else {
         // Free: the whole 6x6; P+ = 0 and G = identity
-        const double b[6] = {tau[0] - z.w.x, tau[1] - z.w.y, tau[2] - z.w.z,
-                             tau[3] - z.v.x, tau[4] - z.v.y, tau[5] - z.v.z};
+        const double b[6] = {ep(0, z.w.x), ep(1, z.w.y), ep(2, z.w.z), ep(3, z.v.x), ep(4, z.v.y), ep(5, z.v.z)};
         const bool bad = solve6(P, b, g);
-        z.w = {tau[0], tau[1], tau[2]}; z.v = {tau[3], tau[4], tau[5]};
+        z.w = {ta(0), ta(1), ta(2)}; z.v = {ta(3), ta(4), ta(5)};
 #pragma unroll
         for (int k = 0; k < 6; ++k) { P.M.a[k] = 0; P.J.a[k] = 0; }
 #pragma unroll
@@ -438,9 +493,11 @@ template <int T> TDJ void add_bias(const art& P, wf& z, const d3& aw, const d3& 
         z.v = z.v + mulsym(P.M, av);
     }
 }
-// P+, z+ from J axes to F axes
-template <int T> TDJ void to_F(const Jnt<T>& J, art& P, wf& z) {
-    z.w = J.fromJ(z.w); z.v = J.fromJ(z.v);
+// P+, z+ from J axes to F axes (TAU: with applied mobility forces; without, a
+// Ball transmits no moment)
+template <int T, bool TAU> TDJ void to_F(const Jnt<T>& J, art& P, wf& z) {
+    if constexpr (T != BALL || TAU) z.w = J.fromJ(z.w);
+    z.v = J.fromJ(z.v);
     double* F = P.F;
     if constexpr (T == PIN) {
         planar<0, 1>(P.M, J.c0, J.s0);
@@ -472,15 +529,20 @@ template <int T> TDJ void to_J(const Jnt<T>& J, art& P, wf& z) {
     z.w = J.fromB(z.w); z.v = J.fromB(z.v);
 }
 // P+, z+ from F axes at F's origin to the parent's M frame
-template <int T, bool IDF, class PA> TDJ void to_parent(const PA& C, art& P, wf& z, const d3& r) {
+template <int T, bool IDF, bool TAU, class PA> TDJ void to_parent(const PA& C, art& P, wf& z, const d3& r) {
     if constexpr (!IDF) {
         dm R; for (int i = 0; i < 9; ++i) R.a[i] = C[JC_R + i];
         P.M = rot(R, P.M);
         if constexpr (T != BALL) { P.J = rot(R, P.J); rot(R, P.F); }
-        z.w = mul(R, z.w); z.v = mul(R, z.v);
+        if constexpr (T != BALL || TAU) z.w = mul(R, z.w);
+        z.v = mul(R, z.v);
     }
-    if constexpr (T == BALL) shift_mass(P, r); else shift(P, r);
-    z.w = z.w + cross(r, z.v);
+    if constexpr (T == BALL) shift_mass(P, r);
+    else if constexpr (T == PIN && IDF) shift_pin(P, r);
+    else if constexpr (T == UNIVERSAL && IDF) shift_universal(P, r);
+    else shift(P, r);
+    if constexpr (T == BALL && !TAU) z.w = cross(r, z.v);
+    else z.w = z.w + cross(r, z.v);
 }
 // P and z of the rigid body itself added (M axes)
 template <class PA> TDJ void add_body(const PA& C, art& P) {
@@ -503,7 +565,7 @@ TDJ art zero_art() { art P; for (int k = 0; k < 6; ++k) { P.M.a[k] = 0; P.J.a[k]
 // with the body added, the joint eliminated and the rest taken to the
 // parent's M frame; w: the body's angular velocity in, its parent's out.
 // z already holds minus the applied force.  root: nothing is handed on.
-template <int T, bool IDF, class PA>
+template <int T, bool IDF, bool TAU, class PA>
 TDJ bool in_body(const PA& C, const Jnt<T>& J, const double* u, const double* tau, art& P, wf& z, d3& w, double* g,
                  bool root) {
     add_body(C, P);
@@ -512,18 +574,18 @@ TDJ bool in_body(const PA& C, const Jnt<T>& J, const double* u, const double* ta
     to_J<T>(J, P, z);
     const d3 wp = J.sub_wrel(J.fromB(w), u);
     bool bad;
-    if constexpr (T == BALL) {
+    if constexpr (T == BALL && TAU) {
         const d3 t = mulT(J.R, d3{tau[0], tau[1], tau[2]});     // given in F
         const double tm[3] = {t.x, t.y, t.z};
-        bad = eliminate<T>(P, z, tm, g);
-    } else bad = eliminate<T>(P, z, tau, g);
+        bad = eliminate<T, TAU>(P, z, tm, g);
+    } else bad = eliminate<T, TAU>(P, z, tau, g);
     if (root) return bad;
     const d3 wF = J.fromJ(wp);
     w = fromF<IDF>(C, wF);
     const d3 r = arm<T, IDF>(C, J);
     if constexpr (T != FREE) add_bias<T>(P, z, J.bias_w(wp, u), bias_v<T, IDF>(C, J, w, wF, r, u));
-    to_F<T>(J, P, z);
-    to_parent<T, IDF>(C, P, z, r);
+    to_F<T, TAU>(J, P, z);
+    to_parent<T, IDF, TAU>(C, P, z, r);
     return bad;
 }
 // One body of the base-to-tip acceleration sweep: A (acceleration of M's

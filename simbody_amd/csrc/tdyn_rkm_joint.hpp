@@ -14,10 +14,10 @@
 //
 // What bounds it.  65,536 chains of 32 bodies are one wavefront per SIMD; a
 // step moves 48 kB per instance between the sweeps (half of it G and DI*eps)
-// at 4.2 TB/s, near what a plain copy reaches, and issues half as many vector
-// instructions as the Ground-frame sweeps did: 0.74 ms per step against
+// at 4.4 TB/s, near what a plain copy reaches, and issues half as many vector
+// instructions as the Ground-frame sweeps did: 0.70 ms per step against
 // 1.43 ms.  A few chains are bound by the latency of one lane's serial sweeps
-// (one 10-link pendulum: 1.1 against 2.2 ms for 45 steps).
+// (one 10-link pendulum: 1.6 against 3.4 ms for 0.1 s at accuracy 1e-8).
 #pragma once
 #include "tdyn_joint.hpp"
 #include "tdyn_rkm_chain.hpp"
@@ -64,7 +64,9 @@ template <int NQ, int D, int G> struct OutB {
 using InC = InB<4, 3>;
 using OutC = OutB<4, 3, 12>;
 
-template <class PA, bool IDF, class Rows, class TC> struct Eval {
+// HASF: with applied body forces (given in Ground, so the bodies' rotations are
+// carried along).
+template <class PA, bool IDF, bool HASF, class Rows, class TC> struct Eval {
     PA prm; const int4* body_j; const int4* body_a;
     int nb, nq;
     Rows sc; TC tc; d3 g; const double* fapp;
@@ -81,7 +83,7 @@ template <class PA, bool IDF, class Rows, class TC> struct Eval {
 #pragma unroll
         for (int k = 0; k < Dim<T>::TC; ++k) tc.put(j.z + k, t[k]);
         w = out_w<T, IDF>(C(b), J, w, u);
-        if (fapp) R = out_R<T, IDF>(C(b), J, R);
+        if constexpr (HASF) R = out_R<T, IDF>(C(b), J, R);
     }
     // MODE 0: the state y itself; 1: the first Merson stage y0 + h/3 f0,
     // stored to st (an attempt after a rejected one)
@@ -146,16 +148,15 @@ template <class PA, bool IDF, class Rows, class TC> struct Eval {
         const PA c = C(b);
         Jnt<T> J;
         J.set(x.q, x.tc);
-        if (fapp) {
+        if constexpr (HASF) {
             const double* f = fapp + 6*b;
             const d3 fm = mulT(R, d3{f[3], f[4], f[5]});
             z.w = z.w - (mulT(R, d3{f[0], f[1], f[2]}) + cross(d3{c[JC_B], c[JC_B + 1], c[JC_B + 2]}, fm));
             z.v = z.v - fm;
             R = in_R<T, IDF>(c, J, R);
         }
-        const double tau[6] = {0, 0, 0, 0, 0, 0};
         double g[Dim<T>::G];
-        (void)in_body<T, IDF>(c, J, x.u, tau, P, z, w, g, b == 1);
+        (void)in_body<T, IDF, false>(c, J, x.u, nullptr, P, z, w, g, b == 1);
         const Rows G = sc.from(j.y);
 #pragma unroll
         for (int k = 0; k < Dim<T>::G; ++k) G(k) = g[k];
@@ -411,9 +412,9 @@ template <bool TILE> TDJ Row<TILE> block_rows(const RkmArgs& a) {
     const size_t off = TILE ? (size_t)blockIdx.x * NVEC * a.ny_max * 64 : (size_t)blockIdx.x * 64;
     return {(TD_GLOBAL double*)a.vec + off, a.L, threadIdx.x * 8u};
 }
-template <class PA, bool IDF, bool TILE, class TC>
-TDJ Eval<PA, IDF, Row<TILE>, TC> make_eval(const RkmArgs& a, int lane, double* lds) {
-    Eval<PA, IDF, Row<TILE>, TC> ev;
+template <class PA, bool IDF, bool HASF, bool TILE, class TC>
+TDJ Eval<PA, IDF, HASF, Row<TILE>, TC> make_eval(const RkmArgs& a, int lane, double* lds) {
+    Eval<PA, IDF, HASF, Row<TILE>, TC> ev;
     const int4 ta = ldi4(a.T.tree_a, 0);
     ev.nb = ta.x; ev.nq = ta.y;
     ev.body_a = a.T.body_a + ta.w; ev.body_j = a.T.body_j + ta.w;
@@ -430,17 +431,17 @@ TDJ Eval<PA, IDF, Row<TILE>, TC> make_eval(const RkmArgs& a, int lane, double* l
         const cdptr g = cptr(a.T.gravity);
         ev.g = {g[0], g[1], g[2]};
     }
-    ev.fapp = a.fapp ? a.fapp + 6*(size_t)a.off.b_off[lane] : nullptr;
+    ev.fapp = HASF ? a.fapp + 6*(size_t)a.off.b_off[lane] : nullptr;
     return ev;
 }
 
-template <class PA, bool IDF, bool TILE, class TC>
+template <class PA, bool IDF, bool HASF, bool TILE, class TC>
 __global__ void __launch_bounds__(64) k_rkm_joint(RkmArgs a) {
     extern __shared__ double lds[];
     const int lane = blockIdx.x * blockDim.x + threadIdx.x;
     if (lane >= a.n_inst) return;
     if (a.status[lane] != 0) return;
-    const auto ev = make_eval<PA, IDF, TILE, TC>(a, lane, lds);
+    const auto ev = make_eval<PA, IDF, HASF, TILE, TC>(a, lane, lds);
     using Rows = Row<TILE>;
     const int4 ta = ldi4(a.T.tree_a, 0);
     const int nb = ta.x, nq = ta.y, nu = ta.z, ny = nq + nu;
@@ -469,7 +470,7 @@ __global__ void __launch_bounds__(64) k_rkm_joint(RkmArgs a) {
         // bases in scalar registers.
         const bool fl = __builtin_amdgcn_readfirstlane(flip ? 1 : 0) != 0;
         const Rows Y = fl ? S1 : S0, Y1 = fl ? S0 : S1;
-        typename Eval<PA, IDF, Rows, TC>::Rk r{Y, Y, ST, rows(R_F0), rows(R_F2), rows(R_F3), Y1, 0.0, 0};
+        typename Eval<PA, IDF, HASF, Rows, TC>::Rk r{Y, Y, ST, rows(R_F0), rows(R_F2), rows(R_F3), Y1, 0.0, 0};
         d3 w; dm R;
         bool ok = false, first = true;
         double t1 = t;
@@ -545,11 +546,11 @@ __global__ void __launch_bounds__(64) k_rkm_joint(RkmArgs a) {
 
 // f = f(y) of the current rollout state into VF0: the derivative the
 // integrator uses.
-template <class PA, bool IDF, bool TILE>
+template <class PA, bool IDF, bool HASF, bool TILE>
 __global__ void __launch_bounds__(64) k_joint_f0(RkmArgs a) {
     const int lane = blockIdx.x * blockDim.x + threadIdx.x;
     if (lane >= a.n_inst) return;
-    const auto ev = make_eval<PA, IDF, TILE, TcG<Row<TILE>>>(a, lane, nullptr);
+    const auto ev = make_eval<PA, IDF, HASF, TILE, TcG<Row<TILE>>>(a, lane, nullptr);
     const Row<TILE> base = block_rows<TILE>(a);
     ev.derivative(base.from(R_Y * a.ny_max), base.from(R_F0 * a.ny_max));
 }
@@ -561,13 +562,17 @@ __global__ void __launch_bounds__(64) k_joint_f0(RkmArgs a) {
 inline bool joint_trig_in_lds(const RkmArgs& a) {
     return a.tc_rows > 0 && a.tc_rows * 64 * 8 <= 163840 / 4;
 }
-template <class PA, bool IDF, bool TILE> hipError_t launch_joint_i(const RkmArgs& a, hipStream_t s, bool f0_only) {
+template <class PA, bool IDF, bool HASF, bool TILE>
+hipError_t launch_joint_f(const RkmArgs& a, hipStream_t s, bool f0_only) {
     using namespace joint;
     const dim3 grd((a.n_inst + 63)/64), blk(64);
-    if (f0_only) k_joint_f0<PA, IDF, TILE><<<grd, blk, 0, s>>>(a);
-    else if (joint_trig_in_lds(a)) k_rkm_joint<PA, IDF, TILE, TcL><<<grd, blk, a.tc_rows * 64 * sizeof(double), s>>>(a);
-    else k_rkm_joint<PA, IDF, TILE, TcG<Row<TILE>>><<<grd, blk, 0, s>>>(a);
+    if (f0_only) k_joint_f0<PA, IDF, HASF, TILE><<<grd, blk, 0, s>>>(a);
+    else if (joint_trig_in_lds(a)) k_rkm_joint<PA, IDF, HASF, TILE, TcL><<<grd, blk, a.tc_rows * 64 * sizeof(double), s>>>(a);
+    else k_rkm_joint<PA, IDF, HASF, TILE, TcG<Row<TILE>>><<<grd, blk, 0, s>>>(a);
     return hipGetLastError();
+}
+template <class PA, bool IDF, bool TILE> hipError_t launch_joint_i(const RkmArgs& a, hipStream_t s, bool f0_only) {
+    return a.fapp ? launch_joint_f<PA, IDF, true, TILE>(a, s, f0_only) : launch_joint_f<PA, IDF, false, TILE>(a, s, f0_only);
 }
 
 } // namespace tdyn

@@ -40,6 +40,7 @@ struct tdyn_server {
     std::vector<char> occupied;
     bool idf = false;      // every model admitted so far has identity joint frames
     bool jidf = true;      // and identity rotations between its joints
+    bool forces = false;   // some admitted request had body forces (without any, adding zeros is left out)
     ~tdyn_server() { if (B) tdyn_batch_destroy(B); }
     int rec_stride() const { return nb * PRM_STRIDE + 3 + nq + nu + 1 + 6 * (nb + 1); }
     RkmArgs rk() const {
@@ -47,6 +48,7 @@ struct tdyn_server {
         a.chain = 1;
         a.prm_lane = prm_lane.p;
         a.idf = idf ? 1 : 0; a.jidf = jidf ? 1 : 0;
+        if (B->precision == 0 && !forces) a.fapp = nullptr;
         return a;
     }
 };
@@ -162,6 +164,7 @@ int tdyn_server_admit(tdyn_server* sv, int n, const tdyn_tree_desc* trees, const
     const int k = std::min<int>(n, (int)sv->free_list.size());
     if (k == 0) return TDYN_OK;
     const int stride = sv->rec_stride();
+    sv->forces = sv->forces || fapp != nullptr;
     HIPCHK(sv->rec_host.reserve((size_t)k * stride));
     HIPCHK(sv->slot_host.reserve(k));
     if (sv->rec_dev.n < (size_t)k * stride) HIPCHK(sv->rec_dev.alloc((size_t)std::max(k, 64) * stride));
@@ -193,7 +196,9 @@ int tdyn_server_admit(tdyn_server* sv, int n, const tdyn_tree_desc* trees, const
     }
     HIPCHK(hipMemcpyAsync(sv->rec_dev.p, sv->rec_host.p, (size_t)k * stride * sizeof(double), hipMemcpyHostToDevice, s));
     HIPCHK(hipMemcpyAsync(sv->slot_dev.p, sv->slot_host.p, (size_t)k * sizeof(int), hipMemcpyHostToDevice, s));
-    HIPCHK(launch_srv_admit(sv->rk(), sv->rec_dev.p, sv->slot_dev.p, k, stride, 0.0, s));
+    RkmArgs ra = sv->rk();
+    ra.fapp = sv->B->fapp.p;
+    HIPCHK(launch_srv_admit(ra, sv->rec_dev.p, sv->slot_dev.p, k, stride, 0.0, s));
     HIPCHK(hipStreamSynchronize(s));
     *n_admitted = k;
     return TDYN_OK;

@@ -77,3 +77,28 @@ def test_rollout(name, accuracy):
         y, s = o.integrate(Y[i], 0.08, accuracy, Fapp=fs[i] if fs else None)
         assert rel_inf(np.concatenate([qs[i], us[i]]), y) < 1e-8, i
         assert (s["attempts"], s["accepted"], s["rejected"], s["projections"]) == tuple(st[i]), (i, st[i], s)
+
+
+def test_large_angles():
+    """Angles near multiples of pi/2, tiny, large, and past the range of the
+    kernels' own sine and cosine: udot of single pendulums and of a
+    Universal against the oracle."""
+    from simbody_amd.matter import MatterBatch, RungeKuttaMerson
+    base = np.array([0.0, 1e-300, 1e-9, 0.5, 1.0, 10.0, 1e3, 1e5, 1048575.9, 1048576.1, 3e7, 1e15])
+    mult = np.pi / 2 * np.array([1.0, 2.0, 3.0, 7.0, 1001.0, 123456.0])
+    qs = np.concatenate([base, -base, mult, np.nextafter(mult, 0), mult + 1e-7, -mult])
+    for types in ([P], [U]):
+        spec = _chain(types, False, 7)
+        n = len(qs)
+        Y = np.zeros((n, spec.nq + spec.nu))
+        Y[:, 0] = qs
+        if types == [U]:
+            Y[:, 1] = qs[::-1]
+        Y[:, spec.nq:] = 0.3
+        batch = MatterBatch([spec], n_instances=n)
+        batch.rollout_begin(batch.pack(Y[:, :spec.nq]), batch.pack(Y[:, spec.nq:]), RungeKuttaMerson(accuracy=1e-6), 0.1)
+        uds = batch.split_u(batch.rollout_derivs()[1])
+        o = OracleModel(spec)
+        for i in range(n):
+            ref = o.realize_acceleration(Y[i, :spec.nq], Y[i, spec.nq:])[0]
+            assert np.abs(uds[i] - ref).max() < 1e-12 * max(1.0, np.abs(ref).max()), (types, qs[i])
