@@ -494,6 +494,11 @@ int tdyn_batch_create(const tdyn_tree_desc* trees, int n_trees, const int32_t* t
     B->h_lane_tree = lane_tree;
     {
     }
+    size_t n_scratch = (size_t)std::max({B->max_rec + 24, B->stream_ok ? B->stream_stride : 0,
+                                         B->stream_ok ? B->group_stride : 0}) * n_instances;
+    // (the joint-frame operators keep G rows in blocks of 64 lanes)
+    if (B->is_chain && tdyn_batch::joint_tiles(n_instances, B->max_nq + B->max_nu))
+        n_scratch = std::max(n_scratch, (size_t)B->g_rows * ((n_instances + 63) / 64 * 64));
     hipError_t e;
     if ((e = B->body_a.upload(B->h_body_a)) != hipSuccess ||
         (e = B->body_b.upload(body_b)) != hipSuccess ||
@@ -515,8 +520,7 @@ int tdyn_batch_create(const tdyn_tree_desc* trees, int n_trees, const int32_t* t
         (e = B->bfs_b.upload(bfs_b)) != hipSuccess ||
         (e = B->prm_bfs.upload(prm_bfs)) != hipSuccess ||
         (e = B->lvl.upload(lvl)) != hipSuccess ||
-        (e = B->scratch.alloc((size_t)std::max({B->max_rec + 24, B->stream_ok ? B->stream_stride : 0,
-                                                B->stream_ok ? B->group_stride : 0}) * n_instances)) != hipSuccess ||
+        (e = B->scratch.alloc(n_scratch)) != hipSuccess ||
         (e = B->op_status.alloc((size_t)n_instances)) != hipSuccess ||
         (e = hipMemset(B->op_status.p, 0, (size_t)n_instances * sizeof(int))) != hipSuccess) {
         delete B;

@@ -153,7 +153,9 @@ struct tdyn_batch {
         std::memset(&a, 0, sizeof(a));
         a.T = tables(); a.tree_of = uniform ? nullptr : tree_of.p; a.n_inst = n_inst; a.L = n_inst;
         a.scratch = scratch.p; a.rec_stride = max_rec + 24; a.off = {q_off.p, u_off.p, b_off.p}; a.inst = permuted ? inst.p : nullptr;
-        a.status = op_status.p; a.jidf = jidf ? 1 : 0;
+        a.status = op_status.p;
+        a.chain = is_chain && scratch.n >= (size_t)g_rows * ((n_inst + 63) / 64 * 64) ? 1 : 0;
+        a.idf = idf ? 1 : 0; a.g_rows = g_rows;
         a.cons_ws = any_cons ? cons_ws.p : nullptr;
         return a;
     }

@@ -172,7 +172,9 @@ struct OpArgs {
     DevTables T;
     const int* tree_of;      // null: every instance uses tree 0
     int n_inst;
-    int jidf;                // as in RkmArgs
+    int chain;               // 1: one serial chain, scratch holds blocks of 64 lanes of its G rows: the
+                             // joint-frame kernels run the operators they have
+    int idf, g_rows;         // as in RkmArgs
     int L;                   // lane pitch of the scratch
     double* scratch;
     int rec_stride;          // doubles of scratch per lane (per-lane record layout of mixed-tree batches)
@@ -200,6 +202,8 @@ struct OpArgs {
     double* out_wit;         // OP_WIT: witness values, WIT_MAX per instance
 };
 hipError_t launch_op(OpKind k, const OpArgs& a, hipStream_t s);
+// The operator on a chain batch in joint frames (false: not one of these).
+bool launch_op_joint(OpKind k, const OpArgs& a, hipStream_t s);
 
 struct RkmArgs {
     DevTables T;

@@ -565,14 +565,18 @@ TDJ art zero_art() { art P; for (int k = 0; k < 6; ++k) { P.M.a[k] = 0; P.J.a[k]
 // with the body added, the joint eliminated and the rest taken to the
 // parent's M frame; w: the body's angular velocity in, its parent's out.
 // z already holds minus the applied force.  root: nothing is handed on.
-template <int T, bool IDF, bool TAU, class PA>
+// VEL: with the velocity terms (else u and w are not read).
+template <int T, bool IDF, bool TAU, bool VEL = true, class PA>
 TDJ bool in_body(const PA& C, const Jnt<T>& J, const double* u, const double* tau, art& P, wf& z, d3& w, double* g,
                  bool root) {
     add_body(C, P);
-    const wf b = gyro(C, w);
-    z.w = z.w + b.w; z.v = z.v + b.v;
+    if constexpr (VEL) {
+        const wf b = gyro(C, w);
+        z.w = z.w + b.w; z.v = z.v + b.v;
+    }
     to_J<T>(J, P, z);
-    const d3 wp = J.sub_wrel(J.fromB(w), u);
+    d3 wp;
+    if constexpr (VEL) wp = J.sub_wrel(J.fromB(w), u);
     bool bad;
     if constexpr (T == BALL && TAU) {
         const d3 t = mulT(J.R, d3{tau[0], tau[1], tau[2]});     // given in F
@@ -580,10 +584,12 @@ TDJ bool in_body(const PA& C, const Jnt<T>& J, const double* u, const double* ta
         bad = eliminate<T, TAU>(P, z, tm, g);
     } else bad = eliminate<T, TAU>(P, z, tau, g);
     if (root) return bad;
-    const d3 wF = J.fromJ(wp);
-    w = fromF<IDF>(C, wF);
     const d3 r = arm<T, IDF>(C, J);
-    if constexpr (T != FREE) add_bias<T>(P, z, J.bias_w(wp, u), bias_v<T, IDF>(C, J, w, wF, r, u));
+    if constexpr (VEL) {
+        const d3 wF = J.fromJ(wp);
+        w = fromF<IDF>(C, wF);
+        if constexpr (T != FREE) add_bias<T>(P, z, J.bias_w(wp, u), bias_v<T, IDF>(C, J, w, wF, r, u));
+    }
     to_F<T, TAU>(J, P, z);
     to_parent<T, IDF, TAU>(C, P, z, r);
     return bad;
@@ -592,12 +598,18 @@ TDJ bool in_body(const PA& C, const Jnt<T>& J, const double* u, const double* ta
 // origin and angular acceleration, the parent's in, the body's out, M axes),
 // w likewise; g as in_body left it.  ud: udot, along the reference's hinge
 // columns.
-template <int T, bool IDF, class PA>
+template <int T, bool IDF, bool VEL = true, class PA>
 TDJ void out_body(const PA& C, const Jnt<T>& J, const double* u, const double* g, wf& A, d3& w, double* ud) {
     const d3 r = arm<T, IDF>(C, J);
-    const d3 wF = toF<IDF>(C, w), wp = J.toJ(wF);
-    d3 av = J.toJ(toF<IDF>(C, A.v + cross(A.w, r))) + bias_v<T, IDF>(C, J, w, wF, r, u);
-    d3 aw = J.toJ(toF<IDF>(C, A.w)) + J.bias_w(wp, u);
+    d3 av = J.toJ(toF<IDF>(C, A.v + cross(A.w, r)));
+    d3 aw = J.toJ(toF<IDF>(C, A.w));
+    d3 wp;
+    if constexpr (VEL) {
+        const d3 wF = toF<IDF>(C, w);
+        wp = J.toJ(wF);
+        av = av + bias_v<T, IDF>(C, J, w, wF, r, u);
+        aw = aw + J.bias_w(wp, u);
+    }
     if constexpr (T == PIN) {
         ud[0] = g[5] - ((g[0]*aw.x + g[1]*aw.y + aw.z) + (g[2]*av.x + g[3]*av.y + g[4]*av.z));
         aw.z += ud[0];
@@ -619,7 +631,71 @@ TDJ void out_body(const PA& C, const Jnt<T>& J, const double* u, const double* g
         aw = {g[0], g[1], g[2]}; av = {g[3], g[4], g[5]};
     }
     A.w = J.toB(aw); A.v = J.toB(av);
-    w = J.toB(J.add_wrel(wp, u));
+    if constexpr (VEL) w = J.toB(J.add_wrel(wp, u));
+}
+// x += H v, x -= H v in J axes (v along the reference's hinge columns)
+template <int T> TDJ void add_hinge(const Jnt<T>& J, wf& x, const double* v, double s) {
+    if constexpr (T == PIN) x.w.z += s*v[0];
+    else if constexpr (T == SLIDER) x.v.x += s*v[0];
+    else if constexpr (T == UNIVERSAL) { x.w.x += s*v[0]; x.w.y += s*v[1]; }
+    else {
+        x.w = x.w + s*J.wrel(v);
+        if constexpr (T == FREE) x.v = x.v + s*d3{v[3], v[4], v[5]};
+    }
+}
+// H^T x, J axes
+template <int T> TDJ void hinge_t(const Jnt<T>& J, const wf& x, double* t) {
+    if constexpr (T == PIN) t[0] = x.w.z;
+    else if constexpr (T == SLIDER) t[0] = x.v.x;
+    else if constexpr (T == UNIVERSAL) { t[0] = x.w.x; t[1] = x.w.y; }
+    else {
+        const d3 f = J.fromJ(x.w);
+        t[0] = f.x; t[1] = f.y; t[2] = f.z;
+        if constexpr (T == FREE) { t[3] = x.v.x; t[4] = x.v.y; t[5] = x.v.z; }
+    }
+}
+// Acceleration (or velocity, with VEL false) of the body from its parent's
+// and v = udot (u) of its joint; and back.
+template <int T, bool IDF, bool VEL, class PA>
+TDJ void out_given(const PA& C, const Jnt<T>& J, const double* u, const double* v, wf& A, d3& w) {
+    const d3 r = arm<T, IDF>(C, J);
+    wf x{J.toJ(toF<IDF>(C, A.w)), J.toJ(toF<IDF>(C, A.v + cross(A.w, r)))};
+    if constexpr (VEL) {
+        const d3 wF = toF<IDF>(C, w), wp = J.toJ(wF);
+        x.v = x.v + bias_v<T, IDF>(C, J, w, wF, r, u);
+        x.w = x.w + J.bias_w(wp, u);
+        w = J.toB(J.add_wrel(wp, u));
+    }
+    add_hinge<T>(J, x, v, 1.0);
+    A.w = J.toB(x.w); A.v = J.toB(x.v);
+}
+template <int T, bool IDF, bool VEL, class PA>
+TDJ void in_given(const PA& C, const Jnt<T>& J, const double* u, const double* v, wf& A, d3& w) {
+    const d3 r = arm<T, IDF>(C, J);
+    wf x{J.fromB(A.w), J.fromB(A.v)};
+    add_hinge<T>(J, x, v, -1.0);
+    if constexpr (VEL) {
+        const d3 wp = J.sub_wrel(J.fromB(w), u), wF = J.fromJ(wp);
+        w = fromF<IDF>(C, wF);
+        x.v = x.v - bias_v<T, IDF>(C, J, w, wF, r, u);
+        x.w = x.w - J.bias_w(wp, u);
+    }
+    A.w = fromF<IDF>(C, J.fromJ(x.w));
+    A.v = fromF<IDF>(C, J.fromJ(x.v)) - cross(A.w, r);
+}
+// A force on the body (M axes) to its parent's M frame.
+template <int T, bool IDF, class PA> TDJ wf in_force(const PA& C, const Jnt<T>& J, const wf& x, const d3& r) {
+    const d3 f = fromF<IDF>(C, J.fromJ(x.v));
+    return {fromF<IDF>(C, J.fromJ(x.w)) + cross(r, f), f};
+}
+// I A (+ velocity terms): the force that gives the rigid body acceleration A
+template <bool VEL, class PA> TDJ wf rigid_force(const PA& C, const wf& A, const d3& w) {
+    const sym I = {{C[JC_I], C[JC_I + 1], C[JC_I + 2], C[JC_I + 3], C[JC_I + 4], C[JC_I + 5]}};
+    const d3 c = {C[JC_C], C[JC_C + 1], C[JC_C + 2]};
+    const double m = C[JC_M];
+    wf f{mulsym(I, A.w) + cross(c, A.v), m*A.v + cross(A.w, c)};
+    if constexpr (VEL) { f.w = f.w + cross(w, mulsym(I, w)); f.v = f.v + centripetal(w, c); }
+    return f;
 }
 
 } // namespace joint

@@ -1691,6 +1691,7 @@ static void launch_op_t(OpKind k, const OpArgs& a, hipStream_t s) {
 }
 hipError_t launch_op(OpKind k, const OpArgs& a, hipStream_t s) {
     if (a.n_inst <= 0) return hipSuccess;
+    if (a.chain && launch_op_joint(k, a, s)) return hipGetLastError();
     if (a.tree_of) launch_op_t<false>(k, a, s); else launch_op_t<true>(k, a, s);
     return hipGetLastError();
 }

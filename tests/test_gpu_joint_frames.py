@@ -102,3 +102,59 @@ def test_large_angles():
         for i in range(n):
             ref = o.realize_acceleration(Y[i, :spec.nq], Y[i, spec.nq:])[0]
             assert np.abs(uds[i] - ref).max() < 1e-12 * max(1.0, np.abs(ref).max()), (types, qs[i])
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_operators(name):
+    spec, batch, Y, q, u, _, _ = _case(name)
+    n = len(Y)
+    rng = np.random.default_rng(len(name))
+    v = rng.normal(size=(n, spec.nu)); f = rng.normal(size=(n, spec.nu))
+    fs = [M.random_body_forces(spec, 3, i) for i in range(n)]
+    V, f_, F_ = batch.pack(v), batch.pack(f), batch.pack(fs)
+    X, Vb, qd, E = batch.realizeKinematics(q, u)
+    E = E.cpu().numpy().reshape(-1, 2)
+    X, Vb, qd = batch.split_b(X, 12), batch.split_b(Vb, 6), batch.split_q(qd)
+    acc, accq = batch.realizeAcceleration(q, u, F_)
+    acc, accq, acc0 = batch.split_u(acc), batch.split_q(accq), batch.split_u(batch.realizeAcceleration(q, u)[0])
+    ud, A, qdd = batch.calcAccelerationIgnoringConstraints(q, u, f_, F_)
+    ud, A, qdd = batch.split_u(ud), batch.split_b(A, 6), batch.split_q(qdd)
+    minv = batch.split_u(batch.multiplyByMInv(q, f_))
+    res = batch.split_u(batch.calcResidualForceIgnoringConstraints(q, u, f_, F_, V))
+    res0 = batch.split_u(batch.calcResidualForceIgnoringConstraints(q, u))
+    mv = batch.split_u(batch.multiplyByM(q, V))
+    jv = batch.split_b(batch.multiplyBySystemJacobian(q, V), 6)
+    jt = batch.split_u(batch.multiplyBySystemJacobianTranspose(q, F_))
+    ba = batch.split_b(batch.calcBodyAccelerationFromUDot(q, u, V), 6)
+    ba0 = batch.split_b(batch.calcBodyAccelerationFromUDot(q, u), 6)
+    abi, abip = (batch.split_b(x, 21) for x in batch.realizeArticulatedBodyInertias(q))
+    cbi = batch.split_b(batch.calcCompositeBodyInertias(q), 10)
+    rf = batch.split_b(batch.calcMobilizerReactionForces(q, u, f_, F_), 6)
+    assert int(batch.op_status().abs().sum()) == 0
+    o = OracleModel(spec)
+    for i in range(0, n, max(1, n // 8)):
+        qi, ui = Y[i, :spec.nq].copy(), Y[i, spec.nq:].copy()
+        k = o.kinematics(qi, ui)
+        oud, oqdd, oA, _ = o.forward(qi, ui, f[i], fs[i])
+        oP, oPP = o.abi(qi, spec.dofs())[:2]
+        r1, rq = o.realize_acceleration(qi, ui, fs[i])[:2]
+        oc = o.composite_inertias(qi)
+        got = dict(X=X, V=Vb, qd=qd, acc=acc, accq=accq, acc0=acc0, ud=ud, A=A, qdd=qdd, minv=minv, res=res, res0=res0,
+                   mv=mv, jv=jv, jt=jt, ba=ba, ba0=ba0, abi=[a[1:] for a in abi], rf=rf)
+        ref = dict(X=k["X_GB"], V=k["V_GB"], qd=k["qdot"], acc=r1, accq=rq, acc0=o.realize_acceleration(qi, ui)[0],
+                   ud=oud, A=oA, qdd=oqdd, minv=o.minv(qi, f[i]), res=o.residual(qi, ui, f[i], fs[i], v[i]),
+                   res0=o.residual(qi, ui), mv=o.multiply_by_m(qi, v[i]), jv=o.jacobian(qi, v[i]),
+                   jt=o.jacobian_transpose(qi, fs[i]), ba=o.body_acceleration(qi, ui, v[i]),
+                   ba0=o.body_acceleration(qi, ui), abi=oP, rf=o.reactions(qi, ui, f[i], fs[i]))
+        for key in got:
+            # scaled by max(|ref|, 1): a lone Pin's velocity torque about its
+            # axis is zero, the oracle's value for it rounding
+            err = np.abs(np.ravel(got[key][i]) - np.ravel(ref[key])).max() / max(1.0, np.abs(ref[key]).max())
+            assert err < (1e-11 if key == "rf" else 1e-12), (key, i, err)
+        # P+ of a lone Free body is zero: compared on P's scale
+        assert np.abs(np.ravel(abip[i][1:]) - np.ravel(oPP)).max() < 1e-12 * np.abs(oP).max(), i
+        c = np.asarray(cbi[i]).reshape(-1, 10)
+        assert np.isinf(c[0, 0]) and np.array_equal(c[0, 1:], oc[0, 1:]), i
+        assert rel_inf(c[1:], oc[1:]) < 1e-12, i
+        for e, key in ((0, "ke"), (1, "pe")):
+            assert abs(E[i, e] - k[key]) <= 1e-12 * max(abs(k[key]), 1.0), (key, i)
