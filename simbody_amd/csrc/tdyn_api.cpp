@@ -186,16 +186,15 @@ int make_rkm_cfg(const tdyn_integrator_cfg* cfg, RkmCfg& c, int& precision) {
 // by size; body-steps/s): 4, 8, 16, 32, 64 lanes for every instance 0.56,
 // 1.06, 1.32, 1.27, 0.95 x 1e8; per instance its widest level in [16, 32]
 // 1.31e8.
-int build_tree_plan(tdyn_batch* b, hipStream_t s) {
-    if (b->tree_lanes == 1) return 0;
+int make_tree_plan(tdyn_batch* b, int tree_lanes, tdyn_batch::Plan& P) {
     const int L = b->n_inst;
     const int64_t resident = std::max(1, tree_group_resident_waves());
-    int gq = b->tree_lanes > 1 ? b->tree_lanes : b->lanes_min;
+    int gq = tree_lanes > 1 ? tree_lanes : b->lanes_min;
     if (gq <= 0) {
         gq = 4;
         while (gq < 16 && (int64_t)L * 2 * gq <= 4 * 64 * resident) gq *= 2;
     }
-    const int gbig = b->tree_lanes > 1 ? gq : std::max(gq, b->lanes_max);
+    const int gbig = tree_lanes > 1 ? gq : std::max(gq, b->lanes_max);
     auto steps = [&](int l, int G) {
         int64_t c = 0;
         for (int w : b->h_tree_lw[b->h_lane_tree[l]]) c += (w + G - 1) / G;
@@ -223,12 +222,24 @@ int build_tree_plan(tdyn_batch* b, hipStream_t s) {
         idx.insert(idx.end(), rest.begin(), rest.end());
     }
     hipError_t e;
-    if ((e = b->plan.upload(plan)) != hipSuccess || (e = b->plan_idx.upload(idx)) != hipSuccess)
+    if ((e = P.waves_of.upload(plan)) != hipSuccess || (e = P.idx.upload(idx)) != hipSuccess)
         return hipfail(e, "tree evaluator plan upload");
-    if (!b->plan_ctr.p && (e = b->plan_ctr.alloc(1)) != hipSuccess) return hipfail(e, "tree evaluator queue counter");
-    b->plan_waves = (int)plan.size();
-    (void)s;
+    if (!P.ctr.p && (e = P.ctr.alloc(1)) != hipSuccess) return hipfail(e, "tree evaluator queue counter");
+    P.waves = (int)plan.size();
     return 0;
+}
+int build_tree_plan(tdyn_batch* b, hipStream_t s) {
+    (void)s;
+    return b->tree_lanes == 1 ? 0 : make_tree_plan(b, b->tree_lanes, b->plan);
+}
+
+int ensure_bfs_consts(tdyn_batch* b, bool ext) {
+    DBuf<double>& t = ext ? b->prm_bfs : b->con_bfs;
+    if (t.p) return TDYN_OK;
+    HIPCHK(t.alloc(b->n_bfs));
+    HIPCHK(launch_bfs_consts(b->tables(), b->n_trees, !ext, t.p, nullptr));
+    HIPCHK(hipStreamSynchronize(nullptr));
+    return TDYN_OK;
 }
 
 int ensure_constraints(tdyn_batch* b) {
@@ -337,8 +348,9 @@ int tdyn_batch_create(const tdyn_tree_desc* trees, int n_trees, const int32_t* t
         }
     }
     B->uniform = ((tree_of_instance == nullptr) || n_trees == 1) && !B->any_rev && !B->any_euler && !B->any_bushing;
-    std::vector<int4> body_b, pre, bfs, bfs_b; std::vector<int> child_idx, lvl; std::vector<double> prm, grav, prm_bfs;
+    std::vector<int4> body_b, pre, bfs, bfs_b; std::vector<int> child_idx, lvl; std::vector<double> prm, grav;
     B->stream_ok = !B->uniform;
+    bool grp_ok = true;          // trees the level-parallel evaluator takes
     std::vector<int> tq(n_trees), tu(n_trees), tnb(n_trees);
     int body_off = 0;
     for (int t = 0; t < n_trees; ++t) {
@@ -377,13 +389,14 @@ int tdyn_batch_create(const tdyn_tree_desc* trees, int n_trees, const int32_t* t
             }
             for (int b = 2; b <= nb; ++b)
                 if (d.mobilizer[b-1] == TDYN_FREE || d.mobilizer[b-1] == TDYN_BUSHING)
-                    B->stream_ok = false;   // a 6-dof body must come first
+                    B->stream_ok = grp_ok = false;   // a 6-dof body must come first
         }
         for (int k = 0; k < 3; ++k) grav.push_back(d.gravity[k]);
         grav.push_back(0.0);
         B->h_tree_a.push_back(make_int4(nb, q, u, body_off));
         // breadth-first order (roots, then each level's children in order):
-        // body, parent's position, first child's position, child count; and
+        // body, parent's position, first position of the children of it or
+        // a later one, child count; and
         // the start of every level
         const int lvl_off = (int)lvl.size();
         size_t prm_base = 0;
@@ -398,23 +411,17 @@ int tdyn_batch_create(const tdyn_tree_desc* trees, int n_trees, const int32_t* t
                 for (int c : ch[b]) { depth[c] = depth[b] + 1; order.push_back(c); }
             }
             starts.push_back(nb);
-            for (int k = 0; k < nb; ++k) {
+            for (int k = 0, first = (int)ch[0].size(); k < nb; ++k) {
                 const int b = order[k], p = d.parent[b - 1];
-                const int first = ch[b].empty() ? 0 : pos[ch[b][0]];
+                first += k > 0 ? (int)ch[order[k - 1]].size() : 0;
                 bfs.push_back(make_int4(b, p == 0 ? -1 : pos[p], first, (int)ch[b].size()));
                 const int4 ba = B->h_body_a[body_off + b - 1];
                 bfs_b.push_back(make_int4(ba.y, ba.z, ba.w, b));
             }
-            // model constants in breadth-first order, in blocks of BW positions
-            // stored constant-major
-            const size_t base = prm_bfs.size();
-            const int BW = tdyn::tgroup::BW;
-            prm_bfs.resize(base + (size_t)tdyn::tgroup::blocks(nb) * BW * PRM_STRIDE, 0.0);
-            for (int k = 0; k < nb; ++k)
-                for (int c = 0; c < PRM_STRIDE; ++c)
-                    prm_bfs[base + (size_t)(k / BW) * PRM_STRIDE * BW + (size_t)c * BW + k % BW] =
-                        prm[(size_t)(body_off + order[k] - 1) * PRM_STRIDE + c];
-            prm_base = base;
+            // room for the constants in breadth-first order (launch_bfs_consts)
+            prm_base = B->n_bfs;
+            B->n_bfs += (size_t)tdyn::tgroup::blocks(nb) * tdyn::tgroup::BW * PRM_STRIDE;
+            if (B->n_bfs > (size_t)INT32_MAX) { delete B; return fail(TDYN_E_SIZE, "batch too large for 32-bit offsets"); }
             int maxw = 0;
             for (size_t k = 0; k + 1 < starts.size(); ++k) maxw = std::max(maxw, starts[k + 1] - starts[k]);
             B->h_tree_maxw.push_back(maxw);
@@ -442,7 +449,7 @@ int tdyn_batch_create(const tdyn_tree_desc* trees, int n_trees, const int32_t* t
         B->max_nq = std::max(B->max_nq, tq[t]); B->max_nu = std::max(B->max_nu, tu[t]);
         B->max_nb = std::max(B->max_nb, tnb[t]);
     }
-    if (q > INT32_MAX || u > INT32_MAX || bb * 21 > INT32_MAX || prm_bfs.size() > (size_t)INT32_MAX) { delete B; return fail(TDYN_E_SIZE, "batch too large for 32-bit offsets"); }
+    if (q > INT32_MAX || u > INT32_MAX || bb * 21 > INT32_MAX) { delete B; return fail(TDYN_E_SIZE, "batch too large for 32-bit offsets"); }
     B->total_q = q; B->total_u = u; B->total_b = bb;
     B->is_chain = B->is_chain && B->uniform;
     B->stream_stride = tdyn::tstream::scratch_doubles(B->dmax, B->max_nb);
@@ -494,8 +501,17 @@ int tdyn_batch_create(const tdyn_tree_desc* trees, int n_trees, const int32_t* t
     B->h_lane_tree = lane_tree;
     {
     }
+    // Forward dynamics of such trees runs level-parallel, one tree in many
+    // instances only where each has its group of 16 lanes at once: 1,024 x 48
+    // bodies 369 -> 74 us, 4,096 x 48 370 -> 99; with more instances the
+    // one-lane kernel fills the device by itself (16,384 x 16 142 us, 234
+    // level-parallel; 65,536 x 48 1,373, 1,482).  Different trees, whose lanes
+    // walk apart in the one-lane kernel, always: 16,384 of 8 to 128 bodies
+    // 3,230 -> 385 us, 65,536 of 8 to 16 1,062 -> 303.
+    grp_ok = grp_ok && !B->is_chain && !B->extended() &&
+             (!B->uniform || (int64_t)n_instances * 16 <= (int64_t)64 * std::max(1, tree_group_resident_waves()));
     size_t n_scratch = (size_t)std::max({B->max_rec + 24, B->stream_ok ? B->stream_stride : 0,
-                                         B->stream_ok ? B->group_stride : 0}) * n_instances;
+                                         B->stream_ok || grp_ok ? B->group_stride : 0}) * n_instances;
     // (the joint-frame operators keep G rows in blocks of 64 lanes)
     if (B->is_chain && tdyn_batch::joint_tiles(n_instances, B->max_nq + B->max_nu))
         n_scratch = std::max(n_scratch, (size_t)B->g_rows * ((n_instances + 63) / 64 * 64));
@@ -518,13 +534,18 @@ int tdyn_batch_create(const tdyn_tree_desc* trees, int n_trees, const int32_t* t
         (e = B->bfs.upload(bfs)) != hipSuccess ||
 
         (e = B->bfs_b.upload(bfs_b)) != hipSuccess ||
-        (e = B->prm_bfs.upload(prm_bfs)) != hipSuccess ||
         (e = B->lvl.upload(lvl)) != hipSuccess ||
         (e = B->scratch.alloc(n_scratch)) != hipSuccess ||
         (e = B->op_status.alloc((size_t)n_instances)) != hipSuccess ||
         (e = hipMemset(B->op_status.p, 0, (size_t)n_instances * sizeof(int))) != hipSuccess) {
         delete B;
         return hipfail(e, "tdyn_batch_create: device allocation/upload");
+    }
+    // operators allocate nothing (they may be captured)
+    if (grp_ok) {
+        int rc = ensure_bfs_consts(B, false);
+        if (!rc) rc = make_tree_plan(B, 0, B->op_plan);
+        if (rc) { delete B; return rc; }
     }
     *out = B;
     return TDYN_OK;
@@ -780,6 +801,10 @@ int tdyn_realize_acceleration(tdyn_batch* b, const double* q, const double* u, c
         HIPCHK(launch_op(OP_FWD_CONS, a, s));
         return TDYN_OK;
     }
+    if (b->op_plan.waves > 0) {
+        HIPCHK(launch_tree_group(b->tree_op(q, u, fapp, udot, qdot), s, true));
+        return TDYN_OK;
+    }
     OpArgs a = b->op();
     a.q = q; a.u = u; a.fbody = fapp; a.out_u = udot; a.out_q = qdot;
     HIPCHK(launch_op(OP_FWD_SYS, a, s));
@@ -947,8 +972,9 @@ static int rollout_begin_impl(tdyn_batch* b, const double* q, const double* u, c
     // rollout in progress.
     b->rollout_ready = false;
     if (grp) {
-        const int rc = build_tree_plan(b, s);
+        int rc = build_tree_plan(b, s);
         if (rc) return rc;
+        if ((rc = ensure_bfs_consts(b, b->extended() || b->known_p))) return rc;
     }
     { const int rc = ensure_rollout_buffers(b, prec); if (rc) return rc; }
     if (b->any_wit) {

@@ -85,7 +85,9 @@ struct tdyn_batch {
     tdyn::host::DBuf<int> child_idx, tree_of, q_off, u_off, b_off;   // per LANE
     tdyn::host::DBuf<int> inst;          // instance of each lane
     bool permuted = false;               // lanes are not in instance order
-    tdyn::host::DBuf<double> prm, gravity, scratch, prm_bfs;
+    tdyn::host::DBuf<double> prm, gravity, scratch;
+    size_t n_bfs = 0;            // doubles of the breadth-first constants
+    tdyn::host::DBuf<double> prm_bfs, con_bfs;   // Ground-frame (extended models and known udot) and joint-frame
     tdyn::host::DBuf<double> prm_j; tdyn::host::DBuf<int4> body_j;   // joint-frame tables (chains)
     bool jidf = false;           // every R_MF is the identity
     int g_rows = 0, tc_rows = 0; // G and trig rows per lane of the joint-frame kernels
@@ -113,8 +115,15 @@ struct tdyn_batch {
     int n_simd = 1024;           // SIMDs of the device (4 per compute unit)
     std::vector<int> h_lane_tree, h_tree_maxw;   // tree of each lane; widest level of each tree
     std::vector<std::vector<int>> h_tree_lw;     // the width of every level of each tree
-    tdyn::host::DBuf<int4> plan; tdyn::host::DBuf<int> plan_idx;   // wavefront plan of the level-parallel evaluator
-    tdyn::host::DBuf<int> plan_ctr;              // its work queue's counter
+    // wavefront plans of the level-parallel evaluator, for rollouts and for
+    // operators: wavefronts, instances in order, the work queue's counter
+    struct Plan {
+        tdyn::host::DBuf<int4> waves_of; tdyn::host::DBuf<int> idx, ctr;
+        int waves = 0;
+        void put(tdyn::RkmArgs& a) const {
+            a.plan = waves_of.p; a.plan_idx = idx.p; a.plan_waves = waves; a.plan_ctr = ctr.p;
+        }
+    } plan, op_plan;
     // holonomic constraints (tdyn_batch_set_constraints): per tree, and their
     // device tables and per-lane workspace (uploaded when changed)
     std::vector<std::vector<tdyn_constraint_desc>> h_cons;
@@ -130,7 +139,6 @@ struct tdyn_batch {
     tdyn::host::DBuf<int> ev_ids, ev_count;
     int ev_cap = 64;
     bool any_wit = false, wit_dirty = false;
-    int plan_waves = 0;
     RkmCfg cfg{};
 
     // Whether the joint-frame kernels keep the rollout state of n chains in
@@ -138,12 +146,13 @@ struct tdyn_batch {
     // unused lanes cost little (64 MiB).
     static bool joint_tiles(int n, int ny) { return n >= 64 || (size_t)tdyn::NVEC * ny * 64 * sizeof(double) <= ((size_t)64 << 20); }
 
+    bool extended() const { return any_rev || any_euler || any_bendstretch || any_bushing; }
     DevTables tables() const {
         DevTables T;
         T.body_a = body_a.p; T.body_b = body_b.p; T.child_idx = child_idx.p; T.prm = prm.p;
         T.prm_j = prm_j.p; T.body_j = body_j.p;
         T.tree_a = tree_a.p; T.tree_b = tree_b.p; T.gravity = gravity.p; T.pre = pre.p; T.bfs = bfs.p; T.lvl = lvl.p;
-        T.bfs_b = bfs_b.p; T.prm_bfs = prm_bfs.p;
+        T.bfs_b = bfs_b.p; T.prm_bfs = prm_bfs.p; T.con_bfs = con_bfs.p;
         T.cons_t = any_cons ? cons_t.p : nullptr; T.cons_a = cons_a.p; T.cons_p = cons_p.p;
         T.wit_t = any_wit ? wit_t.p : nullptr; T.wit_a = wit_a.p; T.wit_p = wit_p.p;
         return T;
@@ -177,12 +186,25 @@ struct tdyn_batch {
         a.idf = (a.chain ? idf : idf_all) ? 1 : 0;
         a.jidf = jidf ? 1 : 0; a.g_rows = g_rows; a.tc_rows = tc_rows;
         a.tile = a.chain && precision == 0 && joint_tiles(n_inst, ny_max) ? 1 : 0;
-        a.ext = (any_rev || any_euler || any_bendstretch || any_bushing || a.presc) ? 1 : 0;
+        a.ext = (extended() || a.presc) ? 1 : 0;
         a.vec_aos = rollout_aos ? 1 : 0;
         a.stream_dmax = dmax;
         a.grp = rollout_aos ? rollout_grp : 0;
-        a.plan = plan.p; a.plan_idx = plan_idx.p; a.plan_waves = plan_waves; a.plan_ctr = plan_ctr.p;
+        plan.put(a);
         if (rollout_aos) a.rec_stride = a.grp ? group_stride : stream_stride;
+        return a;
+    }
+    // Forward dynamics of different trees through the level-parallel evaluator.
+    RkmArgs tree_op(const double* q, const double* u, const double* F, double* udot, double* qdot) const {
+        RkmArgs a;
+        std::memset(&a, 0, sizeof(a));
+        a.T = tables(); a.tree_of = tree_of.p; a.n_inst = n_inst; a.L = n_inst;
+        a.scratch = scratch.p; a.rec_stride = group_stride; a.off = {q_off.p, u_off.p, b_off.p};
+        a.fapp = const_cast<double*>(F);
+        a.idf = idf_all ? 1 : 0;
+        op_plan.put(a);
+        a.op_q = q; a.op_u = u; a.op_qd = qdot; a.op_ud = udot;
+        a.op_status = op_status.p; a.op_inst = permuted ? inst.p : nullptr;
         return a;
     }
 };
@@ -197,6 +219,9 @@ int make_rkm_cfg(const tdyn_integrator_cfg* cfg, RkmCfg& c, int& precision);
 // per-lane time, step, status and statistics, and for precision 1 the
 // mixed path's hand-over rows) for its current sizes.
 int ensure_rollout_buffers(tdyn_batch* b, int precision);
+// The breadth-first constants the level-parallel evaluator needs (ext: the
+// Ground-frame ones), built on the device at first use.
+int ensure_bfs_consts(tdyn_batch* b, bool ext);
 // Uploads the constraint tables and allocates the per-lane workspace when
 // the constraints changed.
 int ensure_constraints(tdyn_batch* b);

@@ -65,6 +65,9 @@ enum {
 // inertia about M's origin (xx yy zz xy xz yz), M axes; the body origin in M;
 // R_MB, the rotation from B to M axes.  (Ground's M frame is Ground.)
 enum { JC_R = 0, JC_L = 9, JC_M = 12, JC_C = 13, JC_I = 16, JC_B = 22, JC_RB = 25 };
+// In the breadth-first blocks of trees (con_bfs): JC_R to JC_B + 2, the Screw
+// pitch, and two spare.
+enum { JC_PITCH = 25, JC_STRIDE = 28 };
 // Hand-over values of one body between the joint-frame sweeps: the entries of
 // G that are not known beforehand with DI*eps, and the trig values of q.
 __host__ __device__ constexpr int jt_g(int t) { return t == UNIVERSAL ? 10 : t == BALL ? 12 : 6; }
@@ -111,12 +114,15 @@ struct DevTables {
     const double* gravity;   // per tree: 4 doubles
     const int4* pre;         // per global body: depth-first preorder of its tree: body, depth, child count, -
     const int4* bfs;         // per global body: breadth-first order of its tree: body, parent's position
-                             // (-1 = Ground), first child's position, child count
+                             // (-1 = Ground), first position of the children of it or a
+                             // later one (the body count if none), child count
     const int* lvl;          // per tree at tree_b.w: level count n, prm_bfs offset, then the n+1 level
                              // starts in bfs order
     const int4* bfs_b;       // per global body, breadth-first order: mobilizer type, qIndex, uIndex, -
-    const double* prm_bfs;   // per tree at lvl[1]: breadth-first positions in blocks of 16, constant k of
-                             // position j at [(j/16)*16*PRM_STRIDE + k*16 + j%16]
+    const double* prm_bfs;   // per tree at lvl[1]: breadth-first positions in blocks of tgroup::BW,
+                             // constant k of position j at [(j/BW)*BW*PRM_STRIDE + k*BW + j%BW]
+    const double* con_bfs;   // the same positions' joint-frame constants, JC_STRIDE per position in such blocks, per
+                             // tree from lvl[1] too
     const int4* cons_t;      // per tree (nullable: no constraints): first constraint, count, rows, -
     const int4* cons_a;      // per constraint: kind, body 1, body 2, -
     const double* cons_p;    // per constraint: station on body 1, station on body 2, rod length (7)
@@ -268,6 +274,12 @@ struct RkmArgs {
     int* ev_ids;             // per lane, ev_cap events: witness, transition (1 falling, 2 rising)
     int* ev_count;           // per lane: events seen since the rollout began (may exceed ev_cap)
     int ev_cap;
+    // level-parallel evaluator, derivative only: packed arguments and results
+    // in place of the rollout's state vectors (nullable; per lane through off)
+    const double *op_q, *op_u;
+    double *op_qd, *op_ud;
+    int* op_status;          // per instance (op_inst: instance of each lane, nullable): 4 where some D is singular
+    const int* op_inst;
 };
 // Per-lane scratch of the streaming tree evaluator (doubles): ST (24 per
 // depth: R p V A of the last body with two or more children seen at that
@@ -340,6 +352,9 @@ hipError_t launch_rkm(const RkmArgs& a, hipStream_t s);
 // Level-parallel tree evaluator (wavefront plan a.plan): rollout steps, or
 // (f0_only) the derivative of the current state.
 hipError_t launch_tree_group(const RkmArgs& a, hipStream_t s, bool f0_only);
+// Breadth-first constants of every tree from prm: the joint-frame ones
+// (joint true, into con_bfs), or prm's own (into prm_bfs).
+hipError_t launch_bfs_consts(const DevTables& T, int n_trees, bool joint, double* out, hipStream_t s);
 // Tree-server slots (pooled tables and state, RkmArgs::pool): admission of n
 // staged requests (per request i: ints at ioff[i], doubles at doff[i], laid
 // out by tdyn_tree_server.cpp) into their slots, and collection of finished

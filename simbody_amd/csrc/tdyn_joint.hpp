@@ -141,8 +141,8 @@ TDJ void shift_universal(art& P, const d3& r) {
 // error 2e-17) and the rest of r to first order: 40 instructions where the
 // library's small-argument path takes 130, under 1 ulp as that is.  One angle
 // per body and derivative made it a sixth of a chain derivative.
-TDJ void sincos_joint(double x, double* sp, double* cp) {
-    if (!(fabs(x) < 1048576.0)) { sincos(x, sp, cp); return; }
+TDJ bool big_angle(double x) { return !(fabs(x) < 1048576.0); }
+TDJ void sincos_small(double x, double* sp, double* cp) {
     const double k = rint(x * 0.6366197723675814);
     const double t = fma(-k, 1.5707963267948966, x);
     const double r = fma(-k, 6.123233995736766e-17, t);
@@ -162,6 +162,10 @@ TDJ void sincos_joint(double x, double* sp, double* cp) {
     const double a = (n & 1) ? cs : sn, b = (n & 1) ? sn : cs;
     *sp = (n & 2) ? -a : a;
     *cp = ((n + 1) & 2) ? -b : b;
+}
+TDJ void sincos_joint(double x, double* sp, double* cp) {
+    if (big_angle(x)) { sincos(x, sp, cp); return; }
+    sincos_small(x, sp, cp);
 }
 
 // ---------------------------------------------------------------------------

@@ -12,6 +12,7 @@
 #include "tdyn_internal.hpp"
 #include "tdyn_math.hpp"
 #include "tdyn_chain.hpp"
+#include "tdyn_joint_const.hpp"
 
 namespace tdyn {
 
@@ -2511,12 +2512,13 @@ __global__ void k_srv_collect(RkmArgs a, const int* slots, int n, double* out, i
 }
 // Tree-server admission: one 64-thread block per request.  ints: nb, nq, nu,
 // body_off, b_off, nquat, rec, grp (1: the level-parallel evaluator), lvl
-// offset, prm_bfs offset, level count, 0, then body_a (4 nb), body_b (4 nb;
+// offset, prm_bfs offset, level count, build (2: Ground frames), then body_a (4 nb), body_b (4 nb;
 // child begin already offset into the pool), child_idx (nb), and for grp
 // bfs (4 nb), bfs_b (4 nb) and the level list (level count + 3).  doubles:
 // prm (nb PRM_STRIDE), gravity (3), q (nq), u (nu), t_end, applied forces
 // (6 (nb+1)), the pool offsets of the slot's vectors and records (2); for
-// grp the breadth-first constants are built here from prm and bfs.
+// grp the breadth-first constants (joint-frame ones but for build 2) are built
+// here from prm and bfs.
 __global__ void __launch_bounds__(64) k_tsrv_admit(RkmArgs a, const int* slots, int n, const long long* ioff,
                                                    const int* ints, const long long* doff, const double* dbl) {
     const int i = blockIdx.x;
@@ -2562,12 +2564,20 @@ __global__ void __launch_bounds__(64) k_tsrv_admit(RkmArgs a, const int* slots, 
     if (grp) {
         // the constants in breadth-first order, blocks of BW positions stored
         // constant-major (padding positions zero), from the staged ones
-        const int BW = tgroup::BW, nd = tgroup::blocks(nb) * BW * PRM_STRIDE;
+        const bool joint = I[11] != 2;
+        const int BW = tgroup::BW, W = joint ? (int)JC_STRIDE : (int)PRM_STRIDE, nd = tgroup::blocks(nb) * BW * W;
         const int* bf = ci + nb;
         double* pb = const_cast<double*>(a.T.prm_bfs) + pbfs_off;
         for (int e = threadIdx.x; e < nd; e += blockDim.x) {
-            const int blk = e / (PRM_STRIDE * BW), r = e % (PRM_STRIDE * BW), c = r / BW, k = blk * BW + r % BW;
-            pb[e] = k < nb ? D[(size_t)(bf[4*k] - 1) * PRM_STRIDE + c] : 0.0;
+            const int blk = e / (W * BW), r = e % (W * BW);
+            const int c = joint ? r / (2*BW) * 2 + r % 2 : r / BW, k = blk * BW + (joint ? r / 2 : r) % BW;
+            double v = 0.0;
+            if (k < nb) {
+                const int b = bf[4*k], p = ba[4*(b - 1)];
+                const double* P = D + (size_t)(b - 1) * PRM_STRIDE;
+                v = joint ? joint::joint_const(P, p ? D + (size_t)(p - 1) * PRM_STRIDE : nullptr, c) : P[c];
+            }
+            pb[e] = v;
         }
     }
     double* y = a.vec + vbase;

@@ -29,6 +29,17 @@
 #include "tdyn_rkm_chain.hpp"
 
 namespace tdyn {
+// Orders the group's memory accesses: what one lane stored before is seen by
+// every lane of the wavefront after (a wavefront's accesses complete in the order issued).
+__device__ __forceinline__ void grp_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+} // namespace tdyn
+#include "tdyn_tree_joint.hpp"
+
+namespace tdyn {
 namespace {
 
 using d3 = v3<double>;
@@ -36,13 +47,6 @@ using dm = m33<double>;
 using dv = sv<double>;
 using da = abi<double>;
 
-// Orders the group's memory accesses: what one lane stored before is seen by
-// every lane of the workgroup (here: the wavefront) after.
-__device__ __forceinline__ void grp_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
 // Sum over the G lanes of a group (aligned lane blocks of G).  The butterfly
 // adds the same pairs in every lane, so all lanes get bitwise the same sum.
 // G is wave-uniform (one G per wavefront).
@@ -91,14 +95,13 @@ struct PZS {
 // hand-overs of passes 1 and 3 through the same frontier measured slower:
 // the records those passes write are read back by later passes anyway.)
 constexpr int kFrontierFields = 30;
-constexpr size_t kFrontierBytes = 64 * 2 * kFrontierFields * sizeof(double);
 
-template <int IDF>
+// The Ground-frame evaluator: models with reversed mobilizers, Euler-angle
+// Balls and Frees, BendStretch or Bushing bodies, and known udot.
 struct GroupEval {
-    // IDF: 0 general joint frames, 1 identity frames at the joints, 2 general
-    // frames with reversed mobilizers or Euler-angle Balls and Frees
-    using PA = std::conditional_t<IDF == 1, chain::IdF<PrmS>,
-                                  std::conditional_t<IDF == 2, chain::ExtF<PrmS>, PrmS>>;
+    static constexpr int kFields = kFrontierFields;
+    static constexpr bool kFused = false;
+    using PA = chain::ExtF<PrmS>;
     using VR = tstream::LaneVec;
     int nb, nq, nlev, l, G;
     double* lf;        // this group's LDS frontier (2 x 30 x G doubles)
@@ -116,8 +119,8 @@ struct GroupEval {
         }
         return VR{a.vec + ((size_t)v * a.L + inst) * a.ny_max};
     }
-    __device__ GroupEval(const RkmArgs& a, int inst, int tr, int lane_in_group, int lanes, double* frontier)
-        : l(lane_in_group), G(lanes), lf(frontier) {
+    __device__ GroupEval(const RkmArgs& a, int inst, int tr, int lane_in_group, int lanes, int group)
+        : l(lane_in_group), G(lanes), lf(joint::lds_frontier + (size_t)group * 2 * kFields * lanes) {
         const int4 ta = ldi4(a.T.tree_a, tr);
         nb = ta.x; nq = ta.y;
         const int body_off = ta.w;
@@ -128,7 +131,7 @@ struct GroupEval {
         const double* g = a.T.gravity + 4*tr;
         grav = V3(g[0], g[1], g[2]);
         fapp = a.fapp ? a.fapp + 6*(size_t)a.off.b_off[inst] : nullptr;
-        pm = (IDF == 2 && a.presc) ? a.presc + a.off.b_off[inst] : nullptr;
+        pm = a.presc ? a.presc + a.off.b_off[inst] : nullptr;
         uk = pm ? a.udot_known + a.off.u_off[inst] : nullptr;
         free0 = ldi4(a.T.body_a, body_off).y == FREE;
     }
@@ -199,9 +202,9 @@ struct GroupEval {
         }
         for (; j < e; j += G) f(TyTag<GEN>{}, j);
     }
-    __device__ __forceinline__ void derivs(const VR& y, const VR& f) const {
+    __device__ __forceinline__ bool derivs(const joint::QU& yy, const joint::QUW& ff) const {
         using namespace chain;
-        const VR fu{f.p + nq};
+        const VR y{const_cast<double*>(yy.q)}, f{ff.q}, fu{ff.u};
         for (int lev = 0; lev < nlev; ++lev) {
             each(lev, [&](auto tag, int j) {
                 constexpr int TY = decltype(tag)::value;
@@ -228,7 +231,7 @@ struct GroupEval {
                 Pre<double> x;
                 load<TY, false>(x, y, bt, st);
                 const double* ukn = nullptr;      // known udot (extended build only)
-                if constexpr (IDF == 2) { if (pm && pm[bt.w]) ukn = uk + bt.z; }
+                if (pm && pm[bt.w]) ukn = uk + bt.z;
                 da PP; dv zp = svzero<double>(); d3 phic = zero3<double>();
                 if (e.w > 0) {
                     // children's P+ and z+, shifted to this body, in child order
@@ -289,6 +292,7 @@ struct GroupEval {
             });
             grp_sync();
         }
+        return false;
     }
 };
 
@@ -296,16 +300,16 @@ struct GroupEval {
 // loop of the other tree evaluators, RungeKuttaMersonIntegratorRep.cpp:
 // 80-160 and AbstractIntegratorRep.cpp:448-502), its vector work split over
 // the group.  l: the lane's index in the group.
-template <int IDF>
-__device__ __forceinline__ void grp_instance(const RkmArgs& a, int inst, int l, int G, double* frontier) {
+template <class EV>
+__device__ __forceinline__ void grp_instance(const RkmArgs& a, int inst, int l, int G, int grp) {
     const int tr = a.tree_of[inst];
-    const GroupEval<IDF> ev(a, inst, tr, l, G, frontier);
+    const EV ev(a, inst, tr, l, G, grp);
     const int4 ta = ldi4(a.T.tree_a, tr);
     const int nb = ta.x, nq = ta.y, nu = ta.z, ny = nq + nu;
     const int4* body_a = a.T.body_a + ta.w;
     const int nquat = ldi4(a.T.tree_b, tr).y;
     using VR = tstream::LaneVec;
-    auto rows = [&](int v) { return GroupEval<IDF>::vrow(a, v, inst); };
+    auto rows = [&](int v) { return GroupEval::vrow(a, v, inst); };
     const VR Y = rows(VY), F0 = rows(VF0), FA = rows(VFA), FB = rows(VFB), YS = rows(VYS),
              Y1 = rows(VY1), YT = rows(VYT), YE = rows(VYE);
 
@@ -319,6 +323,7 @@ __device__ __forceinline__ void grp_instance(const RkmArgs& a, int inst, int l, 
     int attempts = a.stats[4*inst], accepted = a.stats[4*inst+1], rejected = a.stats[4*inst+2],
         projections = a.stats[4*inst+3];
     int status = 0, steps = 0;
+    bool ready = false;      // the evaluator has passed on the angular velocities at Y (or Y1, at a step's end)
 
     // error norm at y1 (IntegratorRep.h:454-523, calcRelativeScaling :644-655),
     // RMS or (setUseInfinityNorm) the largest magnitude
@@ -368,7 +373,32 @@ __device__ __forceinline__ void grp_instance(const RkmArgs& a, int inst, int l, 
             if (!(t1 > t)) { status = -3; break; }
             if (++attempts > cfg.max_attempts) { status = -2; break; }
             const double h = t1 - t;
-            for (int st = s0; st < 5; ++st) {
+            if constexpr (EV::kFused) {
+                // A sweep forms the next stage's state and its angular
+                // velocities; after the last stage these are the next step's.
+                if (s0 == 1) {
+                    for (int k = l; k < ny; k += G) YT(k) = Y(k) + (h/3)*F0(k);
+                    grp_sync();
+                }
+#pragma unroll 1
+                for (int st = s0 == 1 || !ready ? s0 - 1 : s0, hold = st < s0; st < 5; ++st, hold = 0) {
+                    // (hold: before stage s0, at its state)
+                    const int c = hold ? s0 : st;
+                    const double* in = c == 0 ? Y.p : c == 4 ? YS.p : YT.p;
+                    joint::Next n;
+                    n.y = hold ? in : Y.p; n.f0 = c == 0 ? Y.p : F0.p; n.v = c < 3 ? Y.p : c == 3 ? FA.p : FB.p;
+                    n.k = hold ? nullptr : c == 0 ? F0.p : c == 2 ? FA.p : c == 3 ? FB.p : nullptr;
+                    n.out = hold ? YE.p : c == 3 ? YS.p : c == 4 ? Y1.p : YT.p;
+                    n.err = c == 4 ? YE.p : nullptr;
+                    n.c0 = c == 0 ? 0.0 : 1.0; n.cv = c < 3 ? 0.0 : c == 3 ? -3.0 : 4.0;
+                    n.ck = c == 2 ? 3.0 : c == 3 ? 4.0 : 1.0;
+                    n.H = h / (c == 0 ? 3 : c == 2 ? 8 : c == 3 ? 2 : 6);
+                    n.hold = hold;
+                    if (!hold) ev.inward(joint::QU{in, in + nq});
+                    ev.template outward<true>(joint::QU{in, in + nq}, joint::QUW{}, n);
+                }
+                ready = true;
+            } else for (int st = s0; st < 5; ++st) {
                 VR in = Y, out = F0;
                 if (st == 1) {
                     for (int k = l; k < ny; k += G) YT(k) = Y(k) + (h/3)*F0(k);
@@ -384,10 +414,10 @@ __device__ __forceinline__ void grp_instance(const RkmArgs& a, int inst, int l, 
                     in = YS; out = FA;
                 }
                 grp_sync();
-                ev.derivs(in, out);
+                ev.derivs(joint::QU{in.p, in.p + nq}, joint::QUW{out.p, out.p + nq});
             }
             s0 = 1;
-            for (int k = l; k < ny; k += G) {
+            if constexpr (!EV::kFused) for (int k = l; k < ny; k += G) {
                 const double y1 = Y(k) + (h/6)*((F0(k) + 4*FB(k)) + FA(k));
                 Y1(k) = y1;
                 YE(k) = 0.2 * fabs(y1 - YS(k));
@@ -410,6 +440,7 @@ __device__ __forceinline__ void grp_instance(const RkmArgs& a, int inst, int l, 
                 if (qe > projLimit) converged = false;
                 else if (qe > consTol || cfg.force_proj) {
                     ++projections;
+                    ready = false;
                     for (int b = l; b < nb; b += G) {
                         const int4 ba = ldi4(body_a, b);
                         // quaternions only (a Free body flagged PRM_EULER holds angles)
@@ -457,22 +488,30 @@ __device__ __forceinline__ void grp_instance(const RkmArgs& a, int inst, int l, 
 // on 16,384 trees: the groups' steps fall out of phase and the wavefront
 // runs the union of their paths.)  An instance's arithmetic does not depend
 // on the group or wavefront that runs it.
-template <int IDF, bool F0>
-__device__ __forceinline__ void run_instance(const RkmArgs& a, int inst, int l, int G, double* frontier) {
+template <class EV, bool F0>
+__device__ __forceinline__ void run_instance(const RkmArgs& a, int inst, int l, int G, int grp) {
     if constexpr (F0) {
-        const GroupEval<IDF> ev(a, inst, a.tree_of[inst], l, G, frontier);
-        ev.derivs(GroupEval<IDF>::vrow(a, VY, inst), GroupEval<IDF>::vrow(a, VF0, inst));
+        const int tr = a.tree_of[inst];
+        const EV ev(a, inst, tr, l, G, grp);
+        if (a.op_q) {
+            const int qo = a.off.q_off[inst], uo = a.off.u_off[inst];
+            const bool bad = ev.derivs(joint::QU{a.op_q + qo, a.op_u + uo}, joint::QUW{a.op_qd ? a.op_qd + qo : nullptr, a.op_ud + uo});
+            const unsigned long long any = __ballot(bad), mine = G == 64 ? ~0ull : ((1ull << G) - 1);
+            if (l == 0) a.op_status[a.op_inst ? a.op_inst[inst] : inst] = (any >> threadIdx.x) & mine ? 4 : 0;
+        } else {
+            const int nq = ldi4(a.T.tree_a, tr).y;
+            double *y = GroupEval::vrow(a, VY, inst).p, *f = GroupEval::vrow(a, VF0, inst).p;
+            ev.derivs(joint::QU{y, y + nq}, joint::QUW{f, f + nq});
+        }
     } else {
         if (a.status[inst] != 0) return;
-        grp_instance<IDF>(a, inst, l, G, frontier);
+        grp_instance<EV>(a, inst, l, G, grp);
     }
 }
-template <int IDF, bool F0>
+template <class EV, bool F0>
 __device__ __forceinline__ void plan_wave(const RkmArgs& a, int G, int start, int count, int kind) {
-    extern __shared__ double lds_frontier[];
     const int lg = __builtin_ctz((unsigned)G);
     const int grp = threadIdx.x >> lg, l = threadIdx.x & (G - 1);
-    double* frontier = lds_frontier + (size_t)grp * 2 * kFrontierFields * G;
     const int leader = threadIdx.x & ~(G - 1);
     // (one call site of the evaluator for both kinds)
     int k = grp;
@@ -482,17 +521,17 @@ __device__ __forceinline__ void plan_wave(const RkmArgs& a, int G, int start, in
             k = __shfl(k, leader, 64);
         }
         if (k >= count) break;
-        run_instance<IDF, F0>(a, a.plan_idx[start + k], l, G, frontier);
+        run_instance<EV, F0>(a, a.plan_idx[start + k], l, G, grp);
         if (kind == 0) break;
     }
 }
 // One build for every G (4 to 64, a power of two, the same in the whole
 // wavefront): one copy of the evaluator's code serves all wavefronts.
-template <int IDF, bool F0>
+template <class EV, bool F0>
 __global__ void __launch_bounds__(64) k_rkm_plan(RkmArgs a) {
     const int4 w = a.plan[blockIdx.x];
     const int G = __builtin_amdgcn_readfirstlane(w.x);
-    plan_wave<IDF, F0>(a, G, __builtin_amdgcn_readfirstlane(w.y), __builtin_amdgcn_readfirstlane(w.z),
+    plan_wave<EV, F0>(a, G, __builtin_amdgcn_readfirstlane(w.y), __builtin_amdgcn_readfirstlane(w.z),
                        __builtin_amdgcn_readfirstlane(w.w));
 }
 __global__ void k_zero_int(int* p, int n) {
@@ -501,25 +540,49 @@ __global__ void k_zero_int(int* p, int n) {
 
 } // namespace
 
-// a.idf: every tree's joint frames are identity rotations (Simbody's
-// noR_PF/noX_MB node forms), the frame products are skipped; the results
-// are bitwise those of the general form.  a.ext: some mobilizer is reversed
-// or uses Euler angles, or some bodies have known udot; only that build
-// carries the code for them.
-hipError_t launch_tree_group(const RkmArgs& a, hipStream_t s, bool f0_only) {
-    if (a.n_inst <= 0 || a.plan_waves <= 0) return hipSuccess;
+// a.idf: every R_MF is the identity and the products with it are skipped (the
+// results are bitwise those of the general form).  a.ext: some mobilizer is
+// reversed, uses Euler angles or is a BendStretch or Bushing, or some bodies
+// have known udot: the Ground-frame evaluator.
+template <class EV> static void launch_plan(const RkmArgs& a, hipStream_t s, bool f0_only) {
     const dim3 grd((unsigned)a.plan_waves), blk(64);
+    const size_t lds = 64 * 2 * EV::kFields * sizeof(double);
+    if (f0_only) k_rkm_plan<EV, true><<<grd, blk, lds, s>>>(a);
+    else k_rkm_plan<EV, false><<<grd, blk, lds, s>>>(a);
+}
+hipError_t launch_tree_group(const RkmArgs& a, hipStream_t s, bool f0_only) {
+    using joint::GroupJoint;
+    if (a.n_inst <= 0 || a.plan_waves <= 0) return hipSuccess;
     k_zero_int<<<1, 64, 0, s>>>(a.plan_ctr, a.plan_nctr > 0 ? a.plan_nctr : 1);
-    if (a.ext) {
-        if (f0_only) k_rkm_plan<2, true><<<grd, blk, kFrontierBytes, s>>>(a);
-        else k_rkm_plan<2, false><<<grd, blk, kFrontierBytes, s>>>(a);
-    } else if (a.idf) {
-        if (f0_only) k_rkm_plan<1, true><<<grd, blk, kFrontierBytes, s>>>(a);
-        else k_rkm_plan<1, false><<<grd, blk, kFrontierBytes, s>>>(a);
-    } else {
-        if (f0_only) k_rkm_plan<0, true><<<grd, blk, kFrontierBytes, s>>>(a);
-        else k_rkm_plan<0, false><<<grd, blk, kFrontierBytes, s>>>(a);
+    if (a.ext) launch_plan<GroupEval>(a, s, f0_only);
+    else if (a.idf && a.fapp) launch_plan<GroupJoint<true, true>>(a, s, f0_only);
+    else if (a.idf) launch_plan<GroupJoint<true, false>>(a, s, f0_only);
+    else if (a.fapp) launch_plan<GroupJoint<false, true>>(a, s, f0_only);
+    else launch_plan<GroupJoint<false, false>>(a, s, f0_only);
+    return hipGetLastError();
+}
+
+// One 64-thread block per tree.
+__global__ void __launch_bounds__(64) k_bfs_consts(DevTables T, int joint, double* out) {
+    const int4 ta = T.tree_a[blockIdx.x];
+    const int* lv = T.lvl + T.tree_b[blockIdx.x].w;
+    double* o = out + lv[1];
+    const int BW = tgroup::BW, W = joint ? (int)JC_STRIDE : (int)PRM_STRIDE, n = tgroup::blocks(ta.x) * BW * W;
+    for (int e = threadIdx.x; e < n; e += 64) {
+        const int blk = e / (W * BW), r = e % (W * BW);
+        const int c = joint ? r / (2*BW) * 2 + r % 2 : r / BW, k = blk * BW + (joint ? r / 2 : r) % BW;
+        double v = 0.0;
+        if (k < ta.x) {
+            const int b = T.bfs[ta.w + k].x;
+            const double* P = T.prm + (size_t)(ta.w + b - 1) * PRM_STRIDE;
+            const int p = T.body_a[ta.w + b - 1].x;
+            v = joint ? joint::joint_const(P, p ? T.prm + (size_t)(ta.w + p - 1) * PRM_STRIDE : nullptr, c) : P[c];
+        }
+        o[e] = v;
     }
+}
+hipError_t launch_bfs_consts(const DevTables& T, int n_trees, bool joint, double* out, hipStream_t s) {
+    k_bfs_consts<<<dim3((unsigned)n_trees), dim3(64), 0, s>>>(T, joint ? 1 : 0, out);
     return hipGetLastError();
 }
 
@@ -527,7 +590,8 @@ int tree_group_resident_waves() {
     int dev = 0, cus = 0, per_cu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_rkm_plan<1, false>, 64, kFrontierBytes) != hipSuccess)
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_rkm_plan<joint::GroupJoint<true, true>, false>, 64,
+                                                     64 * 2 * joint::JG_PZ_N * sizeof(double)) != hipSuccess)
         return 1024;
     return std::max(1, cus * per_cu);
 }

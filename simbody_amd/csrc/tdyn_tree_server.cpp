@@ -160,8 +160,8 @@ void tree_tables(const tdyn_tree_desc& d, TreeTables& t, int lanes) {
     t.bfs.reserve(4 * (size_t)nb); t.bfs_b.reserve(4 * (size_t)nb);
     t.build = ext ? 2 : identity_frames(d) ? 1 : 0;
     // breadth-first order (roots, then each level's children in order), as
-    // the batches' tables: body, parent's position, first child's position,
-    // child count; mobilizer, qIndex, uIndex, body; the level starts
+    // the batches' tables: body, parent's position, first position of the
+    // children of it or a later one, child count; mobilizer, qIndex, uIndex, body; the level starts
     std::vector<int>& order = t.order; std::vector<int>& pos = t.pos; std::vector<int>& depth = t.depth;
     order.reserve(nb);
     order.assign(cl.begin() + cs[0], cl.begin() + cs[1]);
@@ -175,9 +175,9 @@ void tree_tables(const tdyn_tree_desc& d, TreeTables& t, int lanes) {
         for (int j = cs[b]; j < cs[b + 1]; ++j) { depth[cl[j]] = depth[b] + 1; order.push_back(cl[j]); }
     }
     t.starts.push_back(nb);
-    for (int k = 0; k < nb; ++k) {
+    for (int k = 0, first = cs[1] - cs[0]; k < nb; ++k) {
         const int b = order[k], p = d.parent[b - 1];
-        const int first = nch(b) == 0 ? 0 : pos[cl[cs[b]]];
+        first += k > 0 ? nch(order[k - 1]) : 0;
         t.bfs.insert(t.bfs.end(), {b, p == 0 ? -1 : pos[p], first, nch(b)});
         t.bfs_b.insert(t.bfs_b.end(), {t.body_a[4*(b-1) + 1], t.body_a[4*(b-1) + 2], t.body_a[4*(b-1) + 3], b});
     }
@@ -221,13 +221,14 @@ struct tdyn_tree_server {
     int resident = 0;             // wavefronts of the level-parallel evaluator the device keeps resident
     int n_grp = 0, n_sweep = 0;   // occupied slots on the level-parallel evaluator / on the tree sweeps
     bool plan_dirty = true;
+    bool forces = false;          // some admitted request had body forces
     int plan_off[3] = {0, 0, 0}, plan_n[3] = {0, 0, 0}, plan_nctr = 0;   // per build: its wavefronts
     RkmArgs rk() const {
         RkmArgs a;
         std::memset(&a, 0, sizeof(a));
         a.T.tree_a = tree_a.p; a.T.tree_b = tree_b.p; a.T.body_a = body_a.p; a.T.body_b = body_b.p;
         a.T.child_idx = child.p; a.T.prm = prm.p; a.T.gravity = gravity.p;
-        a.T.bfs = bfs.p; a.T.bfs_b = bfs_b.p; a.T.lvl = lvl.p; a.T.prm_bfs = prm_bfs.p;
+        a.T.bfs = bfs.p; a.T.bfs_b = bfs_b.p; a.T.lvl = lvl.p; a.T.prm_bfs = prm_bfs.p; a.T.con_bfs = prm_bfs.p;
         a.tree_of = tree_of.p; a.n_inst = slots; a.L = slots;
         a.scratch = heap.p; a.vec = heap.p; a.pool = pool.p; a.pool_grp = pool_grp.p;
         a.off = {zero_off.p, zero_off.p, b_off.p};
@@ -434,7 +435,7 @@ int tdyn_tree_server_admit(tdyn_tree_server* sv, int n, const tdyn_tree_desc* tr
         const int lvl_off = 2 * (int)p.body, pbfs_off = (int)p.body * PRM_STRIDE;
         const int nlev = t.grp ? (int)t.starts.size() - 1 : 0;
         I[0] = t.nb; I[1] = t.nq; I[2] = t.nu; I[3] = body_off; I[4] = (int)p.body; I[5] = t.nquat; I[6] = t.rec;
-        I[7] = t.grp; I[8] = lvl_off; I[9] = pbfs_off; I[10] = nlev; I[11] = 0;
+        I[7] = t.grp; I[8] = lvl_off; I[9] = pbfs_off; I[10] = nlev; I[11] = t.build;
         std::copy(t.body_a.begin(), t.body_a.end(), I + 12);
         int* bb = I + 12 + 4 * t.nb;
         for (int b = 0; b < t.nb; ++b) {
@@ -482,6 +483,7 @@ int tdyn_tree_server_admit(tdyn_tree_server* sv, int n, const tdyn_tree_desc* tr
     // the pinned staging is reused by the next call: wait for the copies
     HIPCHK(hipStreamSynchronize(s));
     sv->plan_dirty = true;
+    sv->forces = sv->forces || fapp != nullptr;
     *n_admitted = k;
     return TDYN_OK;
 }
@@ -500,6 +502,7 @@ int tdyn_tree_server_advance(tdyn_tree_server* sv, int max_steps, hipStream_t s)
             g.grp = 1;
             g.idf = bd == 1 ? 1 : 0;
             g.ext = bd == 2 ? 1 : 0;
+            if (!sv->forces && !g.ext) g.fapp = nullptr;
             g.plan = sv->plan.p + sv->plan_off[bd];
             g.plan_waves = sv->plan_n[bd];
             HIPCHK(launch_tree_group(g, s, false));
