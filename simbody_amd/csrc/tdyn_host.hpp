@@ -4,6 +4,8 @@
 #include "../../include/tdyn.h"
 #include "tdyn_internal.hpp"
 
+#include <thread>
+#include <system_error>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -222,6 +224,31 @@ int ensure_rollout_buffers(tdyn_batch* b, int precision);
 // The breadth-first constants the level-parallel evaluator needs (ext: the
 // Ground-frame ones), built on the device at first use.
 int ensure_bfs_consts(tdyn_batch* b, bool ext);
+// fn(i0, i1) over the pieces of [0, n), on up to 8 threads that end before it
+// returns.  work: bodies it goes through; a thread for each 2,048, below which
+// starting one costs more than it saves (packing takes 50 to 130 ns a body).
+// 2,048 requests of 32 bodies: admission 8.7 -> 2.0 ms; 1,024 of 8 to
+// 64: 3.9 -> 1.7 ms.  A piece whose thread cannot start, or that throws there,
+// is run here.
+template <class Fn> void in_pieces(int n, int64_t work, Fn&& fn) {
+    const int m = (int)std::max<int64_t>(1, std::min<int64_t>({8, n, work / 2048, (int64_t)std::thread::hardware_concurrency()}));
+    auto at = [&](int p) { return (int)((int64_t)n * p / m); };
+    std::thread th[8];
+    bool done[8] = {};
+    for (int p = 1; p < m; ++p) {
+        try {
+            th[p] = std::thread([&, p] {
+                try { fn(at(p), at(p + 1)); done[p] = true; } catch (...) {}
+            });
+        } catch (const std::system_error&) {}
+    }
+    struct Join { std::thread* th; ~Join() { for (int p = 1; p < 8; ++p) if (th[p].joinable()) th[p].join(); } };
+    {
+        const Join join{th};
+        fn(0, at(1));
+    }
+    for (int p = 1; p < m; ++p) if (!done[p]) fn(at(p), at(p + 1));
+}
 // Uploads the constraint tables and allocates the per-lane workspace when
 // the constraints changed.
 int ensure_constraints(tdyn_batch* b);

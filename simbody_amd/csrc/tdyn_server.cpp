@@ -3,6 +3,7 @@
 // integrator state; each slot's own model constants live in per-lane rows
 // (RkmArgs::prm_lane) that the chain evaluator reads instead of the shared
 // table.  Admission and retirement move small pinned host records.
+#include <atomic>
 #include "tdyn_host.hpp"
 
 #include <algorithm>
@@ -141,7 +142,7 @@ int tdyn_server_admit(tdyn_server* sv, int n, const tdyn_tree_desc* trees, const
         return fail(TDYN_E_ARG, "tdyn_server_admit: null argument");
     *n_admitted = 0;
     const int nb = sv->nb, nq = sv->nq, nu = sv->nu;
-    for (int i = 0; i < n; ++i) {
+    auto check = [&](int i) -> int {
         const tdyn_tree_desc& d = trees[i];
         if (d.nb != nb || !d.parent || !d.mobilizer ||
             !std::equal(sv->parent.begin(), sv->parent.end(), d.parent) ||
@@ -157,7 +158,19 @@ int tdyn_server_admit(tdyn_server* sv, int n, const tdyn_tree_desc* trees, const
         const int rc = validate_tree(d, i);
         if (rc) return rc;
         if (!std::isfinite(t_end[i])) return fail(TDYN_E_ARG, "tdyn_server_admit: non-finite t_end");
-    }
+        return TDYN_OK;
+    };
+    // (the first refused request gives the error, from this thread)
+    std::atomic<int> bad{n};
+    in_pieces(n, (int64_t)n * nb, [&](int i0, int i1) {
+        for (int i = i0; i < i1; ++i)
+            if (check(i) != TDYN_OK) {
+                int b = bad.load();
+                while (i < b && !bad.compare_exchange_weak(b, i)) {}
+                return;
+            }
+    });
+    if (bad.load() < n) return check(bad.load());
     // a model with general frames switches the server to the general kernel for good
     for (int i = 0; i < std::min<int>(n, (int)sv->free_list.size()); ++i)
         if (sv->idf && !identity_frames(trees[i])) sv->idf = false;
@@ -169,25 +182,31 @@ int tdyn_server_admit(tdyn_server* sv, int n, const tdyn_tree_desc* trees, const
     HIPCHK(sv->slot_host.reserve(k));
     if (sv->rec_dev.n < (size_t)k * stride) HIPCHK(sv->rec_dev.alloc((size_t)std::max(k, 64) * stride));
     if (sv->slot_dev.n < (size_t)k) HIPCHK(sv->slot_dev.alloc((size_t)std::max(k, 64)));
-    for (int i = 0; i < k; ++i) {
-        double* r = sv->rec_host.p + (size_t)i * stride;
-        const tdyn_tree_desc& d = trees[i];
-        // the FP64 slots run in joint frames, the mixed ones in Ground
-        for (int b = 1; b <= nb; ++b) {
-            double* c = r + (size_t)(b-1) * PRM_STRIDE;
-            if (sv->B->precision == 0) pack_joint_consts(d, b, c); else pack_body_params(d, b, c);
+    std::atomic<bool> jidf{sv->jidf};
+    in_pieces(k, (int64_t)k * nb, [&](int i0, int i1) {
+        for (int i = i0; i < i1; ++i) {
+            double* r = sv->rec_host.p + (size_t)i * stride;
+            const tdyn_tree_desc& d = trees[i];
+            // the FP64 slots run in joint frames, the mixed ones in Ground
+            for (int b = 1; b <= nb; ++b) {
+                double* c = r + (size_t)(b-1) * PRM_STRIDE;
+                if (sv->B->precision == 0) pack_joint_consts(d, b, c); else pack_body_params(d, b, c);
+            }
+            if (sv->B->precision == 0 && !identity_joints(r, nb)) jidf = false;
+            double* x = r + (size_t)nb * PRM_STRIDE;
+            x[0] = d.gravity[0]; x[1] = d.gravity[1]; x[2] = d.gravity[2];
+            x += 3;
+            for (int j = 0; j < nq; ++j) x[j] = q[(size_t)i * nq + j];
+            x += nq;
+            for (int j = 0; j < nu; ++j) x[j] = u[(size_t)i * nu + j];
+            x += nu;
+            x[0] = t_end[i];
+            x += 1;
+            for (int j = 0; j < 6 * (nb + 1); ++j) x[j] = fapp ? fapp[(size_t)i * 6 * (nb + 1) + j] : 0.0;
         }
-        if (sv->B->precision == 0) sv->jidf = sv->jidf && identity_joints(r, nb);
-        double* x = r + (size_t)nb * PRM_STRIDE;
-        x[0] = d.gravity[0]; x[1] = d.gravity[1]; x[2] = d.gravity[2];
-        x += 3;
-        for (int j = 0; j < nq; ++j) x[j] = q[(size_t)i * nq + j];
-        x += nq;
-        for (int j = 0; j < nu; ++j) x[j] = u[(size_t)i * nu + j];
-        x += nu;
-        x[0] = t_end[i];
-        x += 1;
-        for (int j = 0; j < 6 * (nb + 1); ++j) x[j] = fapp ? fapp[(size_t)i * 6 * (nb + 1) + j] : 0.0;
+    });
+    sv->jidf = jidf;
+    for (int i = 0; i < k; ++i) {
         const int slot = sv->free_list.back();
         sv->free_list.pop_back();
         sv->occupied[slot] = 1;

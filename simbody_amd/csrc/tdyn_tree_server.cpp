@@ -13,6 +13,7 @@
 // one.  The slots advance together in one launch of the tree sweeps'
 // Runge-Kutta-Merson kernel (a lane per slot; empty and finished slots are
 // skipped), each with its own step control.
+#include <atomic>
 #include "tdyn_host.hpp"
 
 #include <algorithm>
@@ -377,22 +378,45 @@ int tdyn_tree_server_admit(tdyn_tree_server* sv, int n, const tdyn_tree_desc* tr
     if (!sv || n < 0 || (n > 0 && (!trees || !q || !u || !t_end || !slots)) || !n_admitted)
         return fail(TDYN_E_ARG, "tdyn_tree_server_admit: null argument");
     *n_admitted = 0;
-    for (int i = 0; i < n; ++i) {
+    auto check = [&](int i) -> int {
         const int rc = validate_tree(trees[i], i);
         if (rc) return rc;
         if (!std::isfinite(t_end[i]) || !(t_end[i] > 0.0))
             return fail(TDYN_E_ARG, "tdyn_tree_server_admit: t_end must be positive and finite");
-    }
+        return TDYN_OK;
+    };
+    // (the first refused request gives the error, from this thread)
+    std::atomic<int> bad{n};
+    int64_t bodies = 0;
+    for (int i = 0; i < n; ++i) bodies += std::max(0, trees[i].nb);
+    in_pieces(n, bodies, [&](int i0, int i1) {
+        for (int i = i0; i < i1; ++i)
+            if (check(i) != TDYN_OK) {
+                int b = bad.load();
+                while (i < b && !bad.compare_exchange_weak(b, i)) {}
+                return;
+            }
+    });
+    if (bad.load() < n) return check(bad.load());
     // place requests in order while a slot is free and both pools have room
     std::vector<TreeTables>& tabs = sv->tabs;      // reused: their vectors keep their capacity
     std::vector<Held> place;
     size_t nints = 0, ndbl = 0;
     long long qo = 0, uo = 0, fo = 0;
     std::vector<long long> qoff, uoff, foff;
+    int built = 0;
     for (int i = 0; i < n && (int)place.size() < (int)sv->free_list.size(); ++i) {
-        if (tabs.size() <= place.size()) tabs.emplace_back();
-        TreeTables& t = tabs[place.size()];
-        tree_tables(trees[i], t, sv->lanes);
+        if (i == built) {
+            // the next requests' tables, in blocks: with the pools full few are built in vain
+            built = std::min({n, i + 512, (int)sv->free_list.size()});
+            if (tabs.size() < (size_t)built) tabs.resize(built);
+            int64_t work = 0;
+            for (int j = i; j < built; ++j) work += trees[j].nb;
+            in_pieces(built - i, work, [&](int i0, int i1) {
+                for (int j = i + i0; j < i + i1; ++j) tree_tables(trees[j], tabs[j], sv->lanes);
+            });
+        }
+        const TreeTables& t = tabs[i];
         const long long heapn = t.heap_doubles(), nbe = t.body_entries();
         if (nbe > sv->bodies.cap || heapn > sv->heapA.cap) {
             for (const Held& p : place) { sv->bodies.give(p.body, p.nbody); sv->heapA.give(p.heap, p.nheap); }
@@ -424,12 +448,19 @@ int tdyn_tree_server_admit(tdyn_tree_server* sv, int n, const tdyn_tree_desc* tr
     if (e == hipSuccess && sv->slot_dev.n < (size_t)k) e = sv->slot_dev.alloc(std::max(k, 256));
     if (e != hipSuccess) { undo(); return hipfail(e, "tdyn_tree_server_admit: device staging"); }
     size_t io = 0, dof = 0;
+    int64_t packed = 0;
     for (int i = 0; i < k; ++i) {
+        const TreeTables& t = tabs[i];
+        sv->ioff_h.p[i] = (long long)io; sv->doff_h.p[i] = (long long)dof;
+        io += 12 + 9 * (size_t)t.nb + (t.grp ? 8 * (size_t)t.nb + t.starts.size() + 2 : 0);
+        dof += (size_t)t.nb * PRM_STRIDE + 3 + t.nq + t.nu + 1 + 6 * (size_t)(t.nb + 1) + 2;
+        packed += t.nb;
+    }
+    auto pack = [&](int i) {
         const TreeTables& t = tabs[i];
         const Held& p = place[i];
         const int body_off = (int)p.body + 1;
-        sv->ioff_h.p[i] = (long long)io; sv->doff_h.p[i] = (long long)dof;
-        int* I = sv->ints_h.p + io;
+        int* I = sv->ints_h.p + sv->ioff_h.p[i];
         // the level list and the breadth-first constants sit in the slot's
         // body-pool entries: two ints and PRM_STRIDE doubles per entry
         const int lvl_off = 2 * (int)p.body, pbfs_off = (int)p.body * PRM_STRIDE;
@@ -443,7 +474,6 @@ int tdyn_tree_server_admit(tdyn_tree_server* sv, int n, const tdyn_tree_desc* tr
             bb[4*b+2] = t.body_b[4*b+2]; bb[4*b+3] = t.body_b[4*b+3];
         }
         std::copy(t.child.begin(), t.child.end(), bb + 4 * t.nb);
-        io += 12 + 9 * (size_t)t.nb;
         if (t.grp) {
             int* g = I + 12 + 9 * t.nb;
             std::copy(t.bfs.begin(), t.bfs.end(), g);
@@ -451,9 +481,8 @@ int tdyn_tree_server_admit(tdyn_tree_server* sv, int n, const tdyn_tree_desc* tr
             int* lv = g + 8 * t.nb;
             lv[0] = nlev; lv[1] = pbfs_off;
             std::copy(t.starts.begin(), t.starts.end(), lv + 2);
-            io += 8 * (size_t)t.nb + t.starts.size() + 2;
         }
-        double* D = sv->dbl_h.p + dof;
+        double* D = sv->dbl_h.p + sv->doff_h.p[i];
         for (int b = 1; b <= t.nb; ++b) pack_body_params(trees[i], b, D + (size_t)(b-1) * PRM_STRIDE);
         D += (size_t)t.nb * PRM_STRIDE;
         D[0] = trees[i].gravity[0]; D[1] = trees[i].gravity[1]; D[2] = trees[i].gravity[2];
@@ -465,7 +494,10 @@ int tdyn_tree_server_admit(tdyn_tree_server* sv, int n, const tdyn_tree_desc* tr
         D += 6 * (t.nb + 1);
         // vectors after the records
         D[0] = (double)(p.heap + (t.grp ? tgroup::scratch_doubles(t.nb) : t.rec)); D[1] = (double)p.heap;
-        dof += (size_t)t.nb * PRM_STRIDE + 3 + t.nq + t.nu + 1 + 6 * (size_t)(t.nb + 1) + 2;
+    };
+    in_pieces(k, packed, [&](int i0, int i1) { for (int i = i0; i < i1; ++i) pack(i); });
+    for (int i = 0; i < k; ++i) {
+        const Held& p = place[i];
         if (p.grp) ++sv->n_grp; else ++sv->n_sweep;
         const int slot = sv->free_list.back();
         sv->free_list.pop_back();
