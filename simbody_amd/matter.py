@@ -302,6 +302,8 @@ class MatterBatch:
         _check(lib().tdyn_batch_offsets(self.h, qo.ctypes.data_as(_i32), uo.ctypes.data_as(_i32),
                                         bo.ctypes.data_as(_i32)))
         self.q_off, self.u_off, self.b_off = qo, uo, bo
+        self._constrained = False
+        self._angles = any(getattr(t, "use_euler_angles", False) for t in trees)
 
     def __del__(self):
         if getattr(self, "h", None) is not None and _lib is not None:
@@ -341,6 +343,15 @@ class MatterBatch:
     def _new(self, n):
         return self.torch.zeros(int(n), dtype=self.torch.float64, device=self.device)
 
+    def _out(self, n):
+        """An operator's output, every entry of which its kernel writes (no
+        fill: 5 us each where an operator takes 20 to 70)."""
+        return self.torch.empty(int(n), dtype=self.torch.float64, device=self.device)
+
+    def _out_q(self):
+        """The same of q's size; Ball and Free in angles leave a slot as it is."""
+        return self._new(self.total_q) if self._angles else self._out(self.total_q)
+
     def to_device(self, a):
         return self.torch.as_tensor(np.ascontiguousarray(a, np.float64).reshape(-1), device=self.device)
 
@@ -366,9 +377,9 @@ class MatterBatch:
 
     # ---- SimbodyMatterSubsystem surface -----------------------------------
     def realizeKinematics(self, q, u, want_X=True, want_V=True):
-        X = self._new(12 * self.total_b) if want_X else None
-        V = self._new(6 * self.total_b) if want_V else None
-        qd = self._new(self.total_q); E = self._new(2 * self.n_instances)
+        X = self._out(12 * self.total_b) if want_X else None
+        V = self._out(6 * self.total_b) if want_V else None
+        qd = self._out_q(); E = self._out(2 * self.n_instances)
         _check(lib().tdyn_realize_kinematics(self.h, _ptr(q), _ptr(u), _ptr(X), _ptr(V), _ptr(qd),
                                              _ptr(E), _stream()))
         return X, V, qd, E
@@ -394,15 +405,17 @@ class MatterBatch:
         return E[0::2]
 
     def realizeAcceleration(self, q, u, fapp=None):
-        ud = self._new(self.total_u); qd = self._new(self.total_q)
+        # (a failed constraint solve leaves udot as it is)
+        new = self._new if self._constrained else self._out
+        ud = new(self.total_u); qd = new(self.total_q) if self._constrained else self._out_q()
         _check(lib().tdyn_realize_acceleration(self.h, _ptr(q), _ptr(u), _ptr(fapp), _ptr(ud), _ptr(qd),
                                                _stream()))
         return ud, qd
 
     def calcAccelerationIgnoringConstraints(self, q, u, fmob, F, want_A=True, want_qdotdot=True):
-        ud = self._new(self.total_u)
-        A = self._new(6 * self.total_b) if want_A else None
-        qdd = self._new(self.total_q) if want_qdotdot else None
+        ud = self._out(self.total_u)
+        A = self._out(6 * self.total_b) if want_A else None
+        qdd = self._out_q() if want_qdotdot else None
         _check(lib().tdyn_calc_acceleration_ignoring_constraints(
             self.h, _ptr(q), _ptr(u), _ptr(fmob), _ptr(F), _ptr(ud), _ptr(A), _ptr(qdd), _stream()))
         return ud, A, qdd
@@ -451,6 +464,7 @@ class MatterBatch:
                 arr[i].station1[k] = float(s1[k]); arr[i].station2[k] = float(s2[k])
             arr[i].length = float(ln)
         _check(lib().tdyn_batch_set_constraints(self.h, int(tree), n, arr))
+        self._constrained = self._constrained or n > 0
 
     def calcConstrainedAcceleration(self, q, u, F=None):
         """realize(Acceleration) with constraints: (udot, multipliers
@@ -531,50 +545,50 @@ class MatterBatch:
                                     dtype=self.torch.int32, device=self.device)
 
     def multiplyByMInv(self, q, v, out=None):
-        out = self._new(self.total_u) if out is None else out
+        out = self._out(self.total_u) if out is None else out
         _check(lib().tdyn_multiply_by_m_inv(self.h, _ptr(q), _ptr(v), _ptr(out), _stream()))
         return out
 
     def calcResidualForceIgnoringConstraints(self, q, u, fmob=None, F=None, udot=None):
-        out = self._new(self.total_u)
+        out = self._out(self.total_u)
         _check(lib().tdyn_calc_residual_force_ignoring_constraints(
             self.h, _ptr(q), _ptr(u), _ptr(fmob), _ptr(F), _ptr(udot), _ptr(out), _stream()))
         return out
 
     def realizeArticulatedBodyInertias(self, q, want_plus=True):
-        P = self._new(21 * self.total_b)
-        PP = self._new(21 * self.total_b) if want_plus else None
+        P = self._out(21 * self.total_b)
+        PP = self._out(21 * self.total_b) if want_plus else None
         _check(lib().tdyn_calc_articulated_body_inertias(self.h, _ptr(q), _ptr(P), _ptr(PP), _stream()))
         return P, PP
 
     def calcMobilizerReactionForces(self, q, u, fmob, F):
-        out = self._new(6 * self.total_b)
+        out = self._out(6 * self.total_b)
         _check(lib().tdyn_calc_mobilizer_reaction_forces(self.h, _ptr(q), _ptr(u), _ptr(fmob), _ptr(F),
                                                          _ptr(out), _stream()))
         return out
 
     def multiplyByM(self, q, v, out=None):
         """M v per instance (packed like u)."""
-        out = self._new(self.total_u) if out is None else out
+        out = self._out(self.total_u) if out is None else out
         _check(lib().tdyn_multiply_by_m(self.h, _ptr(q), _ptr(v), _ptr(out), _stream()))
         return out
 
     def multiplyBySystemJacobian(self, q, v, out=None):
         """J v: (nb+1)*6 per instance, Ground's entry zero."""
-        out = self._new(6 * self.total_b) if out is None else out
+        out = self._out(6 * self.total_b) if out is None else out
         _check(lib().tdyn_multiply_by_system_jacobian(self.h, _ptr(q), _ptr(v), _ptr(out), _stream()))
         return out
 
     def multiplyBySystemJacobianTranspose(self, q, F_G, out=None):
         """J^T F_G (packed like u); F_G (nb+1)*6 per instance, Ground ignored."""
-        out = self._new(self.total_u) if out is None else out
+        out = self._out(self.total_u) if out is None else out
         _check(lib().tdyn_multiply_by_system_jacobian_transpose(self.h, _ptr(q), _ptr(F_G), _ptr(out),
                                                                 _stream()))
         return out
 
     def calcBodyAccelerationFromUDot(self, q, u, udot=None, out=None):
         """J udot + JDot u: (nb+1)*6 per instance; udot None means zero."""
-        out = self._new(6 * self.total_b) if out is None else out
+        out = self._out(6 * self.total_b) if out is None else out
         _check(lib().tdyn_calc_body_acceleration_from_udot(self.h, _ptr(q), _ptr(u), _ptr(udot), _ptr(out),
                                                            _stream()))
         return out
@@ -582,7 +596,7 @@ class MatterBatch:
     def calcCompositeBodyInertias(self, q, out=None):
         """(nb+1)*10 per instance: mass, mass center (3), unit inertia about
         the body origin (xx yy zz xy xz yz), in G; Ground first."""
-        out = self._new(10 * self.total_b) if out is None else out
+        out = self._out(10 * self.total_b) if out is None else out
         _check(lib().tdyn_calc_composite_body_inertias(self.h, _ptr(q), _ptr(out), _stream()))
         return out
 
