@@ -30,12 +30,12 @@ FLOPS_PER_BODY_STEP = 9034.59375
 FLOPS_RESID_PER_BODY = 1055.40625
 PEAK_FP64_TFLOPS = 78.6      # MI355X FP64 (vector = matrix) peak
 PEAK_HBM_GBS = 8000.0
-# HBM bytes per body-step of k_rkm_chain on this workload, from rocprofv3
-# FETCH_SIZE / WRITE_SIZE per dispatch (difference of a 10-step and a 1-step
-# launch, over 9 steps x 2,097,152 bodies), each scaled by what the same
+# HBM bytes per body-step of k_rkm_joint on this workload, from rocprofv3
+# FETCH_SIZE / WRITE_SIZE per dispatch (a 16-step launch, over 16 steps x
+# 2,097,152 bodies), each scaled by what the same
 # counter reads for a plain 2 GiB device copy (FETCH x2.0, WRITE x1.0).
-TRAFFIC_FETCH_PER_BODY_STEP = 1592.9
-TRAFFIC_WRITE_PER_BODY_STEP = 1040.3
+TRAFFIC_FETCH_PER_BODY_STEP = 920.4
+TRAFFIC_WRITE_PER_BODY_STEP = 623.7
 
 
 def log(msg):
@@ -528,7 +528,7 @@ def main():
                      "traffic_note": "HBM bytes of the timed launch (rocprofv3 FETCH_SIZE+WRITE_SIZE per "
                                      "body-step, copy-calibrated, x body-steps)",
                      "hbm_gbs": traffic / (ms / 1e3) / 1e9, "hbm_frac": traffic / (ms / 1e3) / 1e9 / PEAK_HBM_GBS,
-                     "flops_per_body_step": FLOPS_PER_BODY_STEP, "kernel": "k_rkm_chain"},
+                     "flops_per_body_step": FLOPS_PER_BODY_STEP, "kernel": "k_rkm_joint"},
         "inverse_dynamics": {"ms": id_ms, "bodies_per_s": n * spec.nb / (id_ms / 1e3),
                              "tflops": FLOPS_RESID_PER_BODY * n * spec.nb / (id_ms / 1e3) / 1e12},
         "wall_s_timed": wall,

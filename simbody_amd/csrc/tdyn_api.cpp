@@ -181,7 +181,8 @@ int make_rkm_cfg(const tdyn_integrator_cfg* cfg, RkmCfg& c, int& precision) {
 // tree's levels of ceil(width / G)); a rollout lasts at least as long as
 // its slowest instance, so with the automatic setting an instance whose
 // estimate exceeds the mean load of a group slot runs first, in a wavefront
-// of its own class with lanes_max lanes.  Measured on 16,384 trees of
+// of its own class with lanes_max lanes.  Measured with the Ground-frame
+// evaluator on 16,384 trees of
 // 8..128 bodies, before the queue (static wavefronts of instances ordered
 // by size; body-steps/s): 4, 8, 16, 32, 64 lanes for every instance 0.56,
 // 1.06, 1.32, 1.27, 0.95 x 1e8; per instance its widest level in [16, 32]
@@ -507,7 +508,7 @@ int tdyn_batch_create(const tdyn_tree_desc* trees, int n_trees, const int32_t* t
     // one-lane kernel fills the device by itself (16,384 x 16 142 us, 234
     // level-parallel; 65,536 x 48 1,373, 1,482).  Different trees, whose lanes
     // walk apart in the one-lane kernel, always: 16,384 of 8 to 128 bodies
-    // 3,230 -> 385 us, 65,536 of 8 to 16 1,062 -> 303.
+    // 3,230 -> 371 us, 65,536 of 8 to 16 1,062 -> 303.
     grp_ok = grp_ok && !B->is_chain && !B->extended() &&
              (!B->uniform || (int64_t)n_instances * 16 <= (int64_t)64 * std::max(1, tree_group_resident_waves()));
     size_t n_scratch = (size_t)std::max({B->max_rec + 24, B->stream_ok ? B->stream_stride : 0,

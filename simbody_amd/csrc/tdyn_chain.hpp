@@ -17,7 +17,9 @@
 //
 // Precision.  K is the scalar of the kinematic recursion (X_GB, V_GB, H,
 // HDot terms), the bias forces (coriolis a, gyroscopic b, gravity, z, z+)
-// and the articulated inertias (P, P+, G).  K = double is the FP64 path.
+// and the articulated inertias (P, P+, G).  K = double is the FP64 form: the
+// split precisions' arithmetic and the padded bodies of the tree evaluators
+// (FP64 chains run in joint frames, tdyn_joint.hpp).
 // K = float is the mixed path; in it D = H^T P H is formed with FP64
 // products and sums and inverted in FP64, G = P H D^-1 is formed in FP64
 // and rounded once, DI*eps and udot are FP64, quaternion normalization is

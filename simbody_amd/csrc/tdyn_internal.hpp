@@ -311,7 +311,8 @@ struct LaneStore {
 // a group, which work on consecutive positions, touch consecutive doubles,
 // while each lane still addresses a record's fields by immediate offsets.
 // Fields: pose R p V (0..17), trig cache (18..21), P+ z+ phi for the parent
-// (22..51), A_GB (52..57), G (58..93, 6 per dof) and DI*eps (94..99).
+// (22..51), A_GB (52..57), G (58..93, 6 per dof) and DI*eps (94..99).  The
+// joint-frame form lays its own fields (JG_*) into the same room.
 namespace tgroup {
 enum { R_POSE = 0, R_TC = 18, R_PZ = 22, R_A = 52, R_G = 58, R_DE = 94, NF = 100, BW = 4 };
 __host__ __device__ inline int blocks(int n) { return (n + BW - 1) / BW; }

@@ -5,8 +5,10 @@
 // as its slowest instance (the largest tree with the most step attempts);
 // splitting each instance over G lanes cuts that instance's time.
 //
-// Each instance's bodies are visited in breadth-first order, one tree level
-// at a time (Simbody's level sweeps, SimbodyMatterSubsystemRep.cpp:
+// Two evaluators: GroupJoint (tdyn_tree_joint.hpp), in joint frames, and
+// GroupEval below, in Ground frames, for reversed mobilizers, Euler angles,
+// BendStretch, Bushing and known udot.  In GroupEval each instance's bodies
+// are visited in breadth-first order, one tree level at a time (Simbody's level sweeps, SimbodyMatterSubsystemRep.cpp:
 // realizeArticulatedBodyInertias / calcTreeForwardDynamicsOperator run the
 // same recursions level by level).  The bodies of a level are dealt to the G
 // lanes round-robin (position j to lane j mod G); the levels are separated

@@ -19,9 +19,10 @@
 // - one sweep inward and one outward per derivative of a rollout: the outward
 //   sweep forms the next stage's state and passes on its angular velocities.
 // 16,384 trees of 8 to 128 bodies with forces, 16 lanes each: realize
-// acceleration 385 us; a rollout derivative 640 us, where the Ground-frame
-// evaluator of three sweeps took 1,100 (8 lanes: 10.7 ms for the rollout that
-// 16 take 8.4 for, as twice the records are in use; 32 lanes 10.5).
+// acceleration 371 us (one lane per tree: 3,230); a rollout derivative 490 us,
+// where the Ground-frame evaluator of three sweeps took 1,000.  With 8 lanes
+// a rollout took 10.7 ms for 8.4 with 16, as twice the records are in use,
+// and with 32 lanes 10.5.
 #pragma once
 #include "tdyn_joint.hpp"
 #include "tdyn_joint_const.hpp"
