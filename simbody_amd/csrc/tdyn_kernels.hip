@@ -2431,7 +2431,8 @@ hipError_t launch_rollout_f0(const RkmArgs& a, hipStream_t s) {
 }
 
 // initialize(): forced quaternion normalization, t and h set.
-__device__ void rkm_init_lane(const RkmArgs& a, int lane, double t0) {
+// k0, nk: this thread's share of the instance (every nk-th body).
+__device__ void rkm_init_lane(const RkmArgs& a, int lane, double t0, int k0 = 0, int nk = 1) {
     const Lane c = make_lane(a.T, a.tree_of, lane, a.L, a.scratch);
     if (a.motion && !a.vec_aos) {
         // prescribed q and u at t0 (initialize: prescribeQ, prescribeU)
@@ -2441,7 +2442,7 @@ __device__ void rkm_init_lane(const RkmArgs& a, int lane, double t0) {
     // (a lane with constraints is projected by k_cons_init instead:
     // projectQ normalizes the quaternions as it projects)
     const bool constrained = a.cons_ws && a.T.cons_t && ldi4(a.T.cons_t, a.tree_of ? a.tree_of[lane] : 0).z > 0;
-    for (int b = 1; b <= c.nb && !constrained; ++b) {
+    for (int b = 1 + k0; b <= c.nb && !constrained; b += nk) {
         const int4 ba = c.ba(b);
         if (ba.y != BALL && ba.y != FREE) continue;
         if (c.prm(b)[PRM_EULER] != 0.0) continue;      // x-y-z angles, not a quaternion
@@ -2456,15 +2457,24 @@ __device__ void rkm_init_lane(const RkmArgs& a, int lane, double t0) {
     double h = hinit != -1 ? hinit : cfg.timescale / 10;
     if (hmin != -1) h = fmax(h, hmin);
     if (hmax != -1) h = fmin(h, hmax);
-    a.t[lane] = t0; a.h[lane] = h; a.status[lane] = 0;
-    for (int k = 0; k < 4; ++k) a.stats[4*lane + k] = 0;
+    if (k0 == 0) {
+        a.t[lane] = t0; a.h[lane] = h; a.status[lane] = 0;
+        for (int k = 0; k < 4; ++k) a.stats[4*lane + k] = 0;
+    }
     // Kahan compensation of the mixed path starts at zero
-    if (a.precision != 0) for (int k = 0; k < c.nq + c.nu; ++k) vec_at(a, VC0, lane, k) = 0.0;
+    if (a.precision != 0) for (int k = k0; k < c.nq + c.nu; k += nk) vec_at(a, VC0, lane, k) = 0.0;
 }
 __global__ void __launch_bounds__(64) k_rkm_init(RkmArgs a, double t0) {
     const int lane = blockIdx.x * blockDim.x + threadIdx.x;
     if (lane >= a.n_inst) return;
     rkm_init_lane(a, lane, t0);
+}
+// The same with 16 lanes per instance, for contiguous state vectors (different
+// trees): one lane each took 202 us for 16,384 trees, a memory round trip per
+// body.
+__global__ void __launch_bounds__(64) k_rkm_init_rows(RkmArgs a, double t0) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i / 16 < a.n_inst) rkm_init_lane(a, i / 16, t0, i % 16, 16);
 }
 
 // Serving slots.  Admission record of one request (doubles): nb*PRM_STRIDE
@@ -2659,7 +2669,8 @@ hipError_t launch_srv_collect(const RkmArgs& a, const int* slots, int n, double*
 
 hipError_t launch_rkm_init(const RkmArgs& a, double t0, hipStream_t s) {
     if (a.n_inst <= 0) return hipSuccess;
-    k_rkm_init<<<dim3((a.n_inst + 63)/64), dim3(64), 0, s>>>(a, t0);
+    if (a.vec_aos) k_rkm_init_rows<<<dim3((a.n_inst + 3)/4), dim3(64), 0, s>>>(a, t0);
+    else k_rkm_init<<<dim3((a.n_inst + 63)/64), dim3(64), 0, s>>>(a, t0);
     return hipGetLastError();
 }
 // initialize() of a lane with constraints (Integrator.cpp:376-377): projectQ
