@@ -123,7 +123,8 @@ struct TreeTables {
 // its lanes from the tree's widest level (8 to 32); 4..64 that many lanes.
 void tree_tables(const tdyn_tree_desc& d, TreeTables& t, int lanes) {
     const int nb = d.nb;
-    t.nb = nb;
+    // (t may hold another tree's tables: every field starts over)
+    t.nb = nb; t.nquat = 0; t.grp = 0; t.build = 0; t.G = 0; t.cost = 0;
     // children of every body (Ground 0 included), in increasing order: the
     // range [cs[b], cs[b+1]) of cl
     std::vector<int>& cs = t.cs; std::vector<int>& cl = t.cl;
@@ -187,7 +188,6 @@ void tree_tables(const tdyn_tree_desc& d, TreeTables& t, int lanes) {
     int G = lanes;
     if (G <= 0) { G = 8; while (G < 32 && G < maxw) G *= 2; }
     t.G = G;
-    t.cost = 0;
     for (size_t k = 0; k + 1 < t.starts.size(); ++k) t.cost += (t.starts[k + 1] - t.starts[k] + G - 1) / G;
 }
 
