@@ -4,9 +4,8 @@
 
 namespace tdyn {
 
-hipError_t launch_chain_fp64_lane(const RkmArgs& a, hipStream_t s, bool f0_only) {
-    return a.jidf ? launch_joint_i<joint::PrmT, true, true>(a, s, f0_only)
-                  : launch_joint_i<joint::PrmT, false, true>(a, s, f0_only);
+hipError_t launch_chain_fp64_lane(const RkmArgs& a, hipStream_t s) {
+    return a.kinds ? launch_joint_slots(a, s) : hipSuccess;
 }
 
 } // namespace tdyn

@@ -63,8 +63,9 @@ enum {
 // doubles per body: R_MF, the rotation from F to the parent's M axes; F's
 // origin in the parent's M frame; mass; mass times the mass center, and the
 // inertia about M's origin (xx yy zz xy xz yz), M axes; the body origin in M;
-// R_MB, the rotation from B to M axes.  (Ground's M frame is Ground.)
-enum { JC_R = 0, JC_L = 9, JC_M = 12, JC_C = 13, JC_I = 16, JC_B = 22, JC_RB = 25 };
+// R_MB, the rotation from B to M axes; in body 1 of a serving slot, its kind
+// (SK_*).  (Ground's M frame is Ground.)
+enum { JC_R = 0, JC_L = 9, JC_M = 12, JC_C = 13, JC_I = 16, JC_B = 22, JC_RB = 25, JC_KIND = 34 };
 // In the breadth-first blocks of trees (con_bfs): JC_R to JC_B + 2, the Screw
 // pitch, and two spare.
 enum { JC_PITCH = 25, JC_STRIDE = 28 };
@@ -211,6 +212,11 @@ hipError_t launch_op(OpKind k, const OpArgs& a, hipStream_t s);
 // The operator on a chain batch in joint frames (false: not one of these).
 bool launch_op_joint(OpKind k, const OpArgs& a, hipStream_t s);
 
+// Kinds of FP64 serving slots, by the request itself: identity rotations
+// between its joints, body forces that are not all zero.  Each has its own
+// build of the rollout.
+enum { SK_IDF = 1, SK_FORCES = 2, SK_N = 4 };
+
 struct RkmArgs {
     DevTables T;
     const int* tree_of;
@@ -243,6 +249,7 @@ struct RkmArgs {
                              // or is a BendStretch
     const double* prm_lane;  // chain evaluator with one model per lane (serving slots), nullable:
                              // row k of lane l at prm_lane[k*L + l], nb*PRM_STRIDE model rows then gravity (3)
+    int kinds;               // FP64 serving slots: a bit for each kind (SK_*) that some slot has
     int vec_aos;             // 1: vectors lane-contiguous (entry k of lane l at ((v*L + l)*ny_max + k)) and
                              // the streaming tree evaluator (batches of different trees)
     int stream_dmax;         // streaming tree evaluator: deepest body of any tree
@@ -338,7 +345,7 @@ hipError_t launch_cons_init(const RkmArgs& a, hipStream_t s);
 int tree_group_resident_waves();
 // Chain-evaluator rollouts (f0_only: only the derivative of the current state)
 hipError_t launch_chain_fp64_batch(const RkmArgs& a, hipStream_t s, bool f0_only);
-hipError_t launch_chain_fp64_lane(const RkmArgs& a, hipStream_t s, bool f0_only);
+hipError_t launch_chain_fp64_lane(const RkmArgs& a, hipStream_t s);   // serving slots of the kinds a.kinds
 hipError_t launch_chain_mixed_batch(const RkmArgs& a, hipStream_t s, bool f0_only);
 hipError_t launch_chain_mixed_lane(const RkmArgs& a, hipStream_t s, bool f0_only);
 // precision 2, 3: FP64 arithmetic, single-precision G (and, 3, trig cache) rows
@@ -347,7 +354,8 @@ inline hipError_t launch_chain_variant(const RkmArgs& a, hipStream_t s, bool f0_
     if (a.precision >= 2 && !a.prm_lane) return launch_chain_split_batch(a, s, f0_only);
     if (a.precision == 1)
         return a.prm_lane ? launch_chain_mixed_lane(a, s, f0_only) : launch_chain_mixed_batch(a, s, f0_only);
-    return a.prm_lane ? launch_chain_fp64_lane(a, s, f0_only) : launch_chain_fp64_batch(a, s, f0_only);
+    if (a.prm_lane) return f0_only ? hipErrorInvalidValue : launch_chain_fp64_lane(a, s);
+    return launch_chain_fp64_batch(a, s, f0_only);
 }
 hipError_t launch_rkm(const RkmArgs& a, hipStream_t s);
 // Level-parallel tree evaluator (wavefront plan a.plan): rollout steps, or

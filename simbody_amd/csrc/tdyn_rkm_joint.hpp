@@ -412,6 +412,10 @@ template <bool TILE> TDJ Row<TILE> block_rows(const RkmArgs& a) {
     const size_t off = TILE ? (size_t)blockIdx.x * NVEC * a.ny_max * 64 : (size_t)blockIdx.x * 64;
     return {(TD_GLOBAL double*)a.vec + off, a.L, threadIdx.x * 8u};
 }
+// The model of this lane's serving slot.
+TDJ PrmT slot_prm(const RkmArgs& a, int nb) {
+    return {(const TD_GLOBAL double*)a.prm_lane + blockIdx.x * ((size_t)nb * PRM_STRIDE + 3) * 64, threadIdx.x * 8u};
+}
 template <class PA, bool IDF, bool HASF, bool TILE, class TC>
 TDJ Eval<PA, IDF, HASF, Row<TILE>, TC> make_eval(const RkmArgs& a, int lane, double* lds) {
     Eval<PA, IDF, HASF, Row<TILE>, TC> ev;
@@ -422,8 +426,7 @@ TDJ Eval<PA, IDF, HASF, Row<TILE>, TC> make_eval(const RkmArgs& a, int lane, dou
     if constexpr (std::is_same<TC, TcL>::value) ev.tc = TcL{lds + threadIdx.x};
     else ev.tc = TC{ev.sc.from(a.g_rows)};
     if constexpr (std::is_same<PA, PrmT>::value) {
-        const size_t rows = (size_t)ta.x * PRM_STRIDE + 3;
-        ev.prm = PrmT{(const TD_GLOBAL double*)a.prm_lane + blockIdx.x * rows * 64, threadIdx.x * 8u};
+        ev.prm = slot_prm(a, ta.x);
         const PrmT gl = ev.prm + (size_t)ta.x * PRM_STRIDE;
         ev.g = {gl[0], gl[1], gl[2]};
     } else {
@@ -436,11 +439,7 @@ TDJ Eval<PA, IDF, HASF, Row<TILE>, TC> make_eval(const RkmArgs& a, int lane, dou
 }
 
 template <class PA, bool IDF, bool HASF, bool TILE, class TC>
-__global__ void __launch_bounds__(64) k_rkm_joint(RkmArgs a) {
-    extern __shared__ double lds[];
-    const int lane = blockIdx.x * blockDim.x + threadIdx.x;
-    if (lane >= a.n_inst) return;
-    if (a.status[lane] != 0) return;
+__device__ __forceinline__ void advance_lane(const RkmArgs& a, int lane, double* lds) {
     const auto ev = make_eval<PA, IDF, HASF, TILE, TC>(a, lane, lds);
     using Rows = Row<TILE>;
     const int4 ta = ldi4(a.T.tree_a, 0);
@@ -544,6 +543,34 @@ __global__ void __launch_bounds__(64) k_rkm_joint(RkmArgs a) {
     a.stats[4*lane] = attempts; a.stats[4*lane+1] = accepted; a.stats[4*lane+2] = rejected; a.stats[4*lane+3] = projections;
 }
 
+template <class PA, bool IDF, bool HASF, bool TILE, class TC>
+__global__ void __launch_bounds__(64) k_rkm_joint(RkmArgs a) {
+    extern __shared__ double lds[];
+    const int lane = blockIdx.x * blockDim.x + threadIdx.x;
+    if (lane >= a.n_inst || a.status[lane] != 0) return;
+    advance_lane<PA, IDF, HASF, TILE, TC>(a, lane, lds);
+}
+// Serving slots of every kind (SK_*) in one launch: a block takes the slots of
+// the blockIdx.y-th kind of a.kinds, so that a request runs in the same code
+// whatever its neighbours are, and different kinds run at the same time (one
+// build for the whole server would be the slowest: general frames with forces).
+template <class TC>
+__global__ void __launch_bounds__(64) k_rkm_joint_slots(RkmArgs a) {
+    extern __shared__ double lds[];
+    const int lane = blockIdx.x * blockDim.x + threadIdx.x;
+    int kind = 0;
+    for (int k = 0, y = blockIdx.y; k < SK_N; ++k)
+        if ((a.kinds >> k & 1) && y-- == 0) kind = k;
+    if (lane >= a.n_inst || a.status[lane] != 0) return;
+    if (slot_prm(a, ldi4(a.T.tree_a, 0).x)[JC_KIND] != (double)kind) return;
+    switch (kind) {
+    case 0:                  advance_lane<PrmT, false, false, true, TC>(a, lane, lds); break;
+    case SK_IDF:             advance_lane<PrmT, true, false, true, TC>(a, lane, lds); break;
+    case SK_FORCES:          advance_lane<PrmT, false, true, true, TC>(a, lane, lds); break;
+    case SK_IDF | SK_FORCES: advance_lane<PrmT, true, true, true, TC>(a, lane, lds); break;
+    }
+}
+
 // f = f(y) of the current rollout state into VF0: the derivative the
 // integrator uses.
 template <class PA, bool IDF, bool HASF, bool TILE>
@@ -569,6 +596,13 @@ hipError_t launch_joint_f(const RkmArgs& a, hipStream_t s, bool f0_only) {
     if (f0_only) k_joint_f0<PA, IDF, HASF, TILE><<<grd, blk, 0, s>>>(a);
     else if (joint_trig_in_lds(a)) k_rkm_joint<PA, IDF, HASF, TILE, TcL><<<grd, blk, a.tc_rows * 64 * sizeof(double), s>>>(a);
     else k_rkm_joint<PA, IDF, HASF, TILE, TcG<Row<TILE>>><<<grd, blk, 0, s>>>(a);
+    return hipGetLastError();
+}
+inline hipError_t launch_joint_slots(const RkmArgs& a, hipStream_t s) {
+    using namespace joint;
+    const dim3 grd((a.n_inst + 63)/64, (unsigned)__builtin_popcount((unsigned)a.kinds)), blk(64);
+    if (joint_trig_in_lds(a)) k_rkm_joint_slots<TcL><<<grd, blk, a.tc_rows * 64 * sizeof(double), s>>>(a);
+    else k_rkm_joint_slots<TcG<Row<true>>><<<grd, blk, 0, s>>>(a);
     return hipGetLastError();
 }
 template <class PA, bool IDF, bool TILE> hipError_t launch_joint_i(const RkmArgs& a, hipStream_t s, bool f0_only) {

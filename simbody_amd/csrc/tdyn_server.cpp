@@ -39,17 +39,17 @@ struct tdyn_server {
     Pinned<int> slot_host, outi_host, status_host;
     std::vector<int> free_list;
     std::vector<char> occupied;
-    bool idf = false;      // every model admitted so far has identity joint frames
-    bool jidf = true;      // and identity rotations between its joints
-    bool forces = false;   // some admitted request had body forces (without any, adding zeros is left out)
+    bool idf = false;      // every model admitted so far has identity joint frames (mixed path)
+    std::vector<signed char> kind;      // FP64: SK_* of each occupied slot
+    int n_kind[SK_N] = {};              // and how many of each there are
     ~tdyn_server() { if (B) tdyn_batch_destroy(B); }
     int rec_stride() const { return nb * PRM_STRIDE + 3 + nq + nu + 1 + 6 * (nb + 1); }
     RkmArgs rk() const {
         RkmArgs a = B->rk();
         a.chain = 1;
         a.prm_lane = prm_lane.p;
-        a.idf = idf ? 1 : 0; a.jidf = jidf ? 1 : 0;
-        if (B->precision == 0 && !forces) a.fapp = nullptr;
+        a.idf = idf ? 1 : 0;
+        for (int k = 0; k < SK_N; ++k) a.kinds |= n_kind[k] > 0 ? 1 << k : 0;
         return a;
     }
 };
@@ -122,6 +122,7 @@ int tdyn_server_create(const tdyn_tree_desc* topology, const tdyn_integrator_cfg
     S->free_list.resize(n);
     for (size_t i = 0; i < n; ++i) S->free_list[i] = (int)(n - 1 - i);    // pop_back gives slot 0 first
     S->occupied.assign(n, 0);
+    S->kind.assign(n, 0);
     *out = S;
     return TDYN_OK;
 }
@@ -177,12 +178,10 @@ int tdyn_server_admit(tdyn_server* sv, int n, const tdyn_tree_desc* trees, const
     const int k = std::min<int>(n, (int)sv->free_list.size());
     if (k == 0) return TDYN_OK;
     const int stride = sv->rec_stride();
-    sv->forces = sv->forces || fapp != nullptr;
     HIPCHK(sv->rec_host.reserve((size_t)k * stride));
     HIPCHK(sv->slot_host.reserve(k));
     if (sv->rec_dev.n < (size_t)k * stride) HIPCHK(sv->rec_dev.alloc((size_t)std::max(k, 64) * stride));
     if (sv->slot_dev.n < (size_t)k) HIPCHK(sv->slot_dev.alloc((size_t)std::max(k, 64)));
-    std::atomic<bool> jidf{sv->jidf};
     in_pieces(k, (int64_t)k * nb, [&](int i0, int i1) {
         for (int i = i0; i < i1; ++i) {
             double* r = sv->rec_host.p + (size_t)i * stride;
@@ -192,7 +191,6 @@ int tdyn_server_admit(tdyn_server* sv, int n, const tdyn_tree_desc* trees, const
                 double* c = r + (size_t)(b-1) * PRM_STRIDE;
                 if (sv->B->precision == 0) pack_joint_consts(d, b, c); else pack_body_params(d, b, c);
             }
-            if (sv->B->precision == 0 && !identity_joints(r, nb)) jidf = false;
             double* x = r + (size_t)nb * PRM_STRIDE;
             x[0] = d.gravity[0]; x[1] = d.gravity[1]; x[2] = d.gravity[2];
             x += 3;
@@ -203,21 +201,23 @@ int tdyn_server_admit(tdyn_server* sv, int n, const tdyn_tree_desc* trees, const
             x[0] = t_end[i];
             x += 1;
             for (int j = 0; j < 6 * (nb + 1); ++j) x[j] = fapp ? fapp[(size_t)i * 6 * (nb + 1) + j] : 0.0;
+            // (Ground's force is not applied)
+            const bool forces = std::any_of(x + 6, x + 6 * (nb + 1), [](double f) { return f != 0.0; });
+            if (sv->B->precision == 0) r[JC_KIND] = (identity_joints(r, nb) ? SK_IDF : 0) + (forces ? SK_FORCES : 0);
         }
     });
-    sv->jidf = jidf;
     for (int i = 0; i < k; ++i) {
         const int slot = sv->free_list.back();
         sv->free_list.pop_back();
         sv->occupied[slot] = 1;
+        sv->kind[slot] = sv->B->precision == 0 ? (signed char)sv->rec_host.p[(size_t)i * stride + JC_KIND] : 0;
+        ++sv->n_kind[(int)sv->kind[slot]];
         sv->slot_host.p[i] = slot;
         slots[i] = slot;
     }
     HIPCHK(hipMemcpyAsync(sv->rec_dev.p, sv->rec_host.p, (size_t)k * stride * sizeof(double), hipMemcpyHostToDevice, s));
     HIPCHK(hipMemcpyAsync(sv->slot_dev.p, sv->slot_host.p, (size_t)k * sizeof(int), hipMemcpyHostToDevice, s));
-    RkmArgs ra = sv->rk();
-    ra.fapp = sv->B->fapp.p;
-    HIPCHK(launch_srv_admit(ra, sv->rec_dev.p, sv->slot_dev.p, k, stride, 0.0, s));
+    HIPCHK(launch_srv_admit(sv->rk(), sv->rec_dev.p, sv->slot_dev.p, k, stride, 0.0, s));
     HIPCHK(hipStreamSynchronize(s));
     *n_admitted = k;
     return TDYN_OK;
@@ -269,6 +269,7 @@ int tdyn_server_collect(tdyn_server* sv, int max_out, int32_t* slots, double* q,
         if (status) status[i] = oi[0];
         if (stats) std::copy(oi + 1, oi + 5, stats + (size_t)i * 4);
         sv->occupied[done[i]] = 0;
+        --sv->n_kind[(int)sv->kind[done[i]]];
         sv->free_list.push_back(done[i]);
     }
     *n_out = k;

@@ -1,0 +1,87 @@
+"""A request's result does not depend on its neighbours' options: with body
+forces or without (or with all of them zero), with identity joint frames or
+general ones, served alone, in a mixed burst, or in flight when a request of
+the other kind is admitted: equal to the bit, in both servers."""
+import numpy as np
+import pytest
+
+from common import ext_trees
+from simbody_amd import models as M
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+TYPES = [M.PIN, M.UNIVERSAL, M.BALL, M.SLIDER, M.PIN, M.BALL, M.UNIVERSAL, M.PIN]
+KINDS = [(False, False), (True, False), (False, True), (True, True)]     # general frames, forces
+
+
+def _requests(tree_server, n=12):
+    specs, F = [], []
+    for i in range(n):
+        general, forces = KINDS[i % 4]
+        t = M.random_tree(70, i, nmin=len(TYPES), nmax=len(TYPES), general_frames=general)
+        if tree_server:
+            t.mobilizer = ext_trees(71 + i, 1, nmin=len(TYPES), nmax=len(TYPES))[0].mobilizer
+            t.mobilizer[-1] = M.SCREW
+            t.pitch = np.full(t.nb, 0.3)
+        else:
+            t.parent = np.arange(len(TYPES), dtype=np.int32)
+            t.mobilizer = np.array(TYPES, np.int32)
+        specs.append(t)
+        f = M.random_body_forces(t, 72, i)
+        F.append(f if forces else np.zeros_like(f))
+    ys = [M.random_state(t, 73, i) for i, t in enumerate(specs)]
+    return specs, [y[0] for y in ys], [y[1] for y in ys], np.linspace(0.2, 0.4, n), F
+
+
+def _server(tree_server, specs):
+    from simbody_amd.matter import RungeKuttaMerson
+    from simbody_amd.serving import Server, TreeServer
+    integ = RungeKuttaMerson(accuracy=1e-5)
+    return TreeServer(integ, 1 << 28, max_slots=64) if tree_server else Server(specs[0], integ, 1 << 28, max_slots=64)
+
+
+def _admit(sv, tree_server, req, ids, with_forces):
+    specs, q, u, t, F = ([x[i] for i in ids] for x in req)
+    f = F if with_forces else None
+    if not tree_server:
+        q, u = np.stack(q), np.stack(u)
+        f = None if f is None else np.stack([x.reshape(-1) for x in f])
+    slots = sv.admit(specs, q, u, np.array(t), f)
+    assert len(slots) == len(ids)
+    return {int(s): i for i, s in zip(ids, slots)}
+
+
+def _finish(sv, tree_server, at, out):
+    for _ in range(10000):
+        if not at:
+            return out
+        sv.advance(3)
+        o = sv.collect()
+        for j, s in enumerate(o["slots"]):
+            y = o["y"][j] if tree_server else np.concatenate([o["q"][j], o["u"][j]])
+            out[at.pop(int(s))] = (np.array(y), tuple(o["stats"][j]))
+    raise AssertionError("requests did not finish")
+
+
+@pytest.mark.parametrize("tree_server", [False, True])
+def test_alone_and_beside_other_kinds(tree_server):
+    req = _requests(tree_server)
+    n = len(req[0])
+    alone = {}
+    for i in range(n):
+        sv = _server(tree_server, req[0])
+        alone.update(_finish(sv, tree_server, _admit(sv, tree_server, req, [i], bool(np.any(req[4][i]))), {}))
+    # one burst of all kinds
+    sv = _server(tree_server, req[0])
+    burst = _finish(sv, tree_server, _admit(sv, tree_server, req, list(range(n)), True), {})
+    # one after the other, each in flight when the next kind comes, on a server that has served all kinds
+    late, at = {}, {}
+    for i in range(n):
+        at.update(_admit(sv, tree_server, req, [i], bool(np.any(req[4][i]))))
+        sv.advance(2)
+    _finish(sv, tree_server, at, late)
+    for i in range(n):
+        for other in (burst, late):
+            assert alone[i][1] == other[i][1], (i, KINDS[i % 4])
+            assert np.array_equal(alone[i][0], other[i][0]), (i, KINDS[i % 4])
