@@ -659,7 +659,7 @@ template <int T> TDJ void hinge_t(const Jnt<T>& J, const wf& x, double* t) {
     }
 }
 // Acceleration (or velocity, with VEL false) of the body from its parent's
-// and v = udot (u) of its joint; and back.
+// and v = udot (u) of its joint.
 template <int T, bool IDF, bool VEL, class PA>
 TDJ void out_given(const PA& C, const Jnt<T>& J, const double* u, const double* v, wf& A, d3& w) {
     const d3 r = arm<T, IDF>(C, J);
@@ -672,20 +672,6 @@ TDJ void out_given(const PA& C, const Jnt<T>& J, const double* u, const double* 
     }
     add_hinge<T>(J, x, v, 1.0);
     A.w = J.toB(x.w); A.v = J.toB(x.v);
-}
-template <int T, bool IDF, bool VEL, class PA>
-TDJ void in_given(const PA& C, const Jnt<T>& J, const double* u, const double* v, wf& A, d3& w) {
-    const d3 r = arm<T, IDF>(C, J);
-    wf x{J.fromB(A.w), J.fromB(A.v)};
-    add_hinge<T>(J, x, v, -1.0);
-    if constexpr (VEL) {
-        const d3 wp = J.sub_wrel(J.fromB(w), u), wF = J.fromJ(wp);
-        w = fromF<IDF>(C, wF);
-        x.v = x.v - bias_v<T, IDF>(C, J, w, wF, r, u);
-        x.w = x.w - J.bias_w(wp, u);
-    }
-    A.w = fromF<IDF>(C, J.fromJ(x.w));
-    A.v = fromF<IDF>(C, J.fromJ(x.v)) - cross(A.w, r);
 }
 // A force on the body (M axes) to its parent's M frame.
 template <int T, bool IDF, class PA> TDJ wf in_force(const PA& C, const Jnt<T>& J, const wf& x, const d3& r) {

@@ -2,12 +2,17 @@
 // (tdyn_joint.hpp): one lane per instance, the sweep state in registers.
 //
 // The record-based sweeps (k_op) write and read 0.7-1.6 kB per body between
-// sweeps.  Here a sweep back along the chain recovers what the sweep out
-// computed (angular velocities, accelerations, rotations) from the tip's
-// values and the joint's own q, u, udot, and the joint angles' sines are
-// formed again, so only forward dynamics keeps anything per body (G and
-// DI*eps, 6 to 12 doubles); the rest of the traffic is the arguments and the
-// results themselves.
+// sweeps.  Here a sweep keeps 6 to 12 doubles per body for the next one (G and
+// DI*eps, or the force on the body), the joint angles' sines are formed again,
+// and rotations are recovered on the way back along the chain; the rest of the
+// traffic is the arguments and the results themselves.
+//
+// Velocities and accelerations are not recovered from the tip's: a slow body's
+// would carry the rounding of a fast outer one's.  So each body's force is
+// formed on the way out, from the body's own acceleration, and kept.  (M v,
+// the residual and the reactions with everything recovered: base torque of a
+// two-link chain off by 7e-10 where the tip is 1e-8 of the link's mass and as
+// much faster.  65,536 x 32 inverse dynamics: 180 us so, 203 as it is.)
 #include "tdyn_joint.hpp"
 
 namespace tdyn {
@@ -37,7 +42,7 @@ struct Tab { int y, q, u, g; };
 // What a sweep needs of one body, loaded one body ahead.
 struct In { double q[7], u[6], v[6], f[6], g[12]; };
 
-enum : unsigned { LD_U = 1, LD_V = 2, LD_TAU = 4, LD_F = 8, LD_G = 16 };
+enum : unsigned { LD_U = 1, LD_V = 2, LD_TAU = 4, LD_F = 8, LD_G = 16, LD_FM = 32 };   // (LD_FM: the force kept, put_force)
 
 template <bool IDF> struct Chain {
     cdptr prm; const int4 *body_a, *body_j;
@@ -79,6 +84,19 @@ template <bool IDF> struct Chain {
 #pragma unroll
             for (int k = 0; k < Dim<T>::G; ++k) x.g[k] = g(k);
         }
+        if constexpr ((W & LD_FM) != 0) {
+            const Blk g = G.from(j.g);
+#pragma unroll
+            for (int k = 0; k < 6; ++k) x.g[k] = g(k);
+        }
+    }
+    // A force on body j (M axes) into its G rows, and out of them again.
+    TDJ void put_force(const Tab& j, const wf& f) const {
+        const Blk g = G.from(j.g);
+        g(0) = f.w.x; g(1) = f.w.y; g(2) = f.w.z; g(3) = f.v.x; g(4) = f.v.y; g(5) = f.v.z;
+    }
+    static TDJ void add_kept(wf& f, const In& x) {
+        f.w = f.w + d3{x.g[0], x.g[1], x.g[2]}; f.v = f.v + d3{x.g[3], x.g[4], x.g[5]};
     }
     template <unsigned W> TDJ void load_any(In& x, int b, const Tab& j) const {
         switch (j.y) {
@@ -193,7 +211,7 @@ __global__ void __launch_bounds__(64) k_cop(OpArgs a) {
         w = zero3<double>(); R = ident<double>();
         const Pk ob = packed(a.out_body, first, 6*(c.nb + 1));
         const bool hasA = OP == OP_FWD_GIVEN && ob, hasR = hasA || OP == OP_REACT;
-        c.template sweep<true, (VEL ? LD_U : 0u) | LD_G>([&](auto t, const In& x, int b, const Tab& j) {
+        c.template sweep<true, (VEL ? LD_U : 0u) | LD_G | (OP == OP_REACT ? LD_F : 0u)>([&](auto t, const In& x, int b, const Tab& j) {
             constexpr int T = decltype(t)::t;
             constexpr int D = Dim<T>::D, NQ = Dim<T>::NQ;
             const cdptr C = c.C(b);
@@ -205,13 +223,13 @@ __global__ void __launch_bounds__(64) k_cop(OpArgs a) {
 #pragma unroll
                 for (int k = 0; k < D; ++k) o(k) = ud[k];
             }
-            if constexpr (OP == OP_REACT) {
-                // udot kept for the sweep back
-                const Blk G = c.G.from(j.g);
-#pragma unroll
-                for (int k = 0; k < D; ++k) G(k) = ud[k];
-            }
             if (hasR) R = out_R<T, IDF>(C, J, R);
+            if constexpr (OP == OP_REACT) {
+                // (G has been read)
+                wf r = rigid_force<true>(C, A, w);
+                if (hasF) { const wf e = c.force_M(C, R, x.f); r.w = r.w - e.w; r.v = r.v - e.v; }
+                c.put_force(j, r);
+            }
             if (hasA) c.put_body(ob.from(6*b), C, R, A, &w);
             if constexpr (OP == OP_FWD_SYS || OP == OP_FWD_GIVEN) {
                 if (!c.oq) return;
@@ -238,17 +256,14 @@ __global__ void __launch_bounds__(64) k_cop(OpArgs a) {
         if constexpr (OP == OP_REACT) {
             // the force through each mobilizer at M, gathered tip to base
             wf f{zero3<double>(), zero3<double>()};
-            c.template sweep<false, LD_U | LD_F | LD_G>([&](auto t, const In& x, int b, const Tab& j) {
+            c.template sweep<false, LD_FM>([&](auto t, const In& x, int b, const Tab& j) {
                 constexpr int T = decltype(t)::t;
                 const cdptr C = c.C(b);
                 const Jnt<T> J = c.template joint_of<T>(x);
-                const wf r = rigid_force<true>(C, A, w);
-                f.w = f.w + r.w; f.v = f.v + r.v;
-                if (hasF) { const wf e = c.force_M(C, R, x.f); f.w = f.w - e.w; f.v = f.v - e.v; }
+                c.add_kept(f, x);
                 const d3 n = mul(R, f.w), l = mul(R, f.v);
                 const Pk o = ob.from(6*b);
                 o(0) = n.x; o(1) = n.y; o(2) = n.z; o(3) = l.x; o(4) = l.y; o(5) = l.z;
-                in_given<T, IDF, true>(C, J, x.u, x.g, A, w);
                 f = in_force<T, IDF>(C, J, wf{J.fromB(f.w), J.fromB(f.v)}, arm<T, IDF>(C, J));
                 R = in_R<T, IDF>(C, J, R);
             });
@@ -263,7 +278,7 @@ __global__ void __launch_bounds__(64) k_cop(OpArgs a) {
         double ke = 0, pe = 0;
         const Pk ob = packed(a.out_body, first, (OP == OP_KIN ? 12 : 6)*(c.nb + 1)),
                  ov = packed(a.out_body2, first, 6*(c.nb + 1));
-        c.template sweep<true, (VEL || OP == OP_KIN ? LD_U : 0u) | (OP != OP_KIN ? LD_V : 0u)>(
+        c.template sweep<true, (VEL || OP == OP_KIN ? LD_U : 0u) | (OP != OP_KIN ? LD_V : 0u) | (OP == OP_RESID ? LD_F : 0u)>(
             [&](auto t, const In& x, int b, const Tab& j) {
                 constexpr int T = decltype(t)::t;
                 const cdptr C = c.C(b);
@@ -271,6 +286,11 @@ __global__ void __launch_bounds__(64) k_cop(OpArgs a) {
                 if constexpr (OP == OP_KIN) p = p + mul(R, arm<T, IDF>(C, J));
                 out_given<T, IDF, VEL>(C, J, x.u, OP == OP_KIN ? x.u : x.v, A, w);
                 if (OUTB || hasF) R = out_R<T, IDF>(C, J, R);
+                if constexpr (OP == OP_RESID || OP == OP_MULM) {
+                    wf r = rigid_force<VEL>(C, A, w);
+                    if (hasF) { const wf e = c.force_M(C, R, x.f); r.w = r.w - e.w; r.v = r.v - e.v; }
+                    c.put_force(j, r);
+                }
                 if constexpr (OP == OP_JAC || OP == OP_BACC) c.put_body(ob.from(6*b), C, R, A, VEL ? &w : nullptr);
                 if constexpr (OP == OP_KIN) {
                     const wf h = rigid_force<false>(C, A, w);
@@ -307,24 +327,17 @@ __global__ void __launch_bounds__(64) k_cop(OpArgs a) {
         }
         if constexpr (OP == OP_RESID || OP == OP_MULM) {
             wf f{zero3<double>(), zero3<double>()};
-            c.template sweep<false, (VEL ? LD_U : 0u) | LD_V | (VEL ? LD_F : 0u)>([&](auto t, const In& x, int b, const Tab& j) {
+            c.template sweep<false, LD_FM>([&](auto t, const In& x, int b, const Tab& j) {
                 constexpr int T = decltype(t)::t;
                 const cdptr C = c.C(b);
                 const Jnt<T> J = c.template joint_of<T>(x);
-                const wf r = rigid_force<VEL>(C, A, w);
-                f.w = f.w + r.w; f.v = f.v + r.v;
-                if (hasF) {
-                    const wf e = c.force_M(C, R, x.f);
-                    f.w = f.w - e.w; f.v = f.v - e.v;
-                    R = in_R<T, IDF>(C, J, R);
-                }
+                c.add_kept(f, x);
                 const wf fj{J.fromB(f.w), J.fromB(f.v)};
                 double tt[Dim<T>::D];
                 hinge_t<T>(J, fj, tt);
                 const Pk o = c.ou.from(j.u), fm = c.tau.from(j.u);
 #pragma unroll
                 for (int k = 0; k < Dim<T>::D; ++k) o(k) = OP == OP_RESID && c.tau ? tt[k] - fm(k) : tt[k];
-                in_given<T, IDF, VEL>(C, J, x.u, x.v, A, w);
                 f = in_force<T, IDF>(C, J, fj, arm<T, IDF>(C, J));
             });
         }

@@ -1,0 +1,135 @@
+"""Badly scaled models and states, each quantity on its own scale: a light fast
+distal link.
+
+Tolerances.  A recursion that forms every body's own values from its parent's
+is off by a few roundings of the quantity's own terms: with chains of three
+bodies and at most 32 terms of rounding 1.1e-16, 1e-13 of an entry's terms
+covers it; where a vector is compared on its largest entry, 1e-12."""
+import numpy as np
+import pytest
+
+from simbody_amd import models as M
+from oracle_ctypes import OracleModel
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+def _planar(mobilizer, masses, parent=None):
+    """Links along x, joints about z at their inner end, mass center halfway;
+    the last body a wheel about its own joint where its mass is negative."""
+    n = len(mobilizer)
+    m = np.abs(np.array(masses, float))
+    com = np.zeros((n, 3)); I = np.zeros((n, 6)); XF = np.tile(M._xform(), (n, 1)); XM = np.tile(M._xform(), (n, 1))
+    parent = np.arange(n) if parent is None else np.array(parent)
+    for b in range(n):
+        if masses[b] > 0:
+            com[b, 0] = 0.5
+            I[b] = m[b] * np.array([0.01, 0.01 + 0.25, 0.02 + 0.25, 0, 0, 0])
+        else:
+            I[b] = m[b] * np.array([0.02, 0.02, 0.04, 0, 0, 0])
+        if parent[b] > 0:
+            XF[b, 9] = 1.0
+    return M.TreeSpec(parent=parent.astype(np.int32), mobilizer=np.array(mobilizer, np.int32), mass=m, com_B=com,
+                      inertia_B=I, X_PF=XF, X_BM=XM)
+
+
+def _residual(spec, q, u, udot):
+    """H^T of the forces that give udot, in extended precision: the recursion
+    in Ground, one hinge axis after the other; and the sum of the magnitudes
+    of the terms that make up each entry."""
+    L = np.longdouble
+    x3 = np.zeros(3, L)
+    R, p, w, al, a = np.eye(3).astype(L), x3, x3, x3, x3         # frame; its origin's acceleration
+    hinges, bodies, qi, ui = [], [], 0, 0
+    for b in range(spec.nb):
+        r = R @ spec.X_PF[b, 9:].astype(L)
+        a = a + np.cross(al, r) + np.cross(w, np.cross(w, r))
+        p = p + r
+        ty = int(spec.mobilizer[b])
+
+        def turn(axis, k, w, al):
+            rate = L(u[k]) * axis
+            return w + rate, al + L(udot[k]) * axis + np.cross(w, rate)
+
+        if ty == M.SLIDER:
+            ax, x = R[:, 0].copy(), L(q[qi])
+            hinges.append((ui, None, ax, len(bodies)))
+            a = a + np.cross(al, x * ax) + np.cross(w, np.cross(w, x * ax)) + 2 * L(u[ui]) * np.cross(w, ax) + L(udot[ui]) * ax
+            p = p + x * ax
+        elif ty == M.BALL:
+            F = R.copy()
+            rate, acc = F @ np.array(u[ui:ui + 3], L), F @ np.array(udot[ui:ui + 3], L)
+            hinges += [(ui + k, p, F[:, k], len(bodies)) for k in range(3)]
+            w, al = w + rate, al + acc + np.cross(w, rate)
+            n = np.array(q[qi:qi + 4], L)
+            c, s = (n / np.sqrt(n @ n))[0], (n / np.sqrt(n @ n))[1:]
+            S = np.array([[0, -s[2], s[1]], [s[2], 0, -s[0]], [-s[1], s[0], 0]], L)
+            R = R @ (np.eye(3) + 2 * c * S + 2 * S @ S)
+        else:
+            for k, i in enumerate([2] if ty == M.PIN else [0, 1]):
+                hinges.append((ui + k, p, R[:, i].copy(), len(bodies)))
+                w, al = turn(R[:, i], ui + k, w, al)
+                c, s = np.cos(L(q[qi + k])), np.sin(L(q[qi + k]))
+                m, n = (i + 1) % 3, (i + 2) % 3
+                T = np.eye(3).astype(L)
+                T[m, m] = T[n, n] = c
+                T[m, n], T[n, m] = -s, s
+                R = R @ T
+        m, cb, I6 = L(spec.mass[b]), spec.com_B[b].astype(L), spec.inertia_B[b].astype(L)
+        I = np.array([[I6[0], I6[3], I6[4]], [I6[3], I6[1], I6[5]], [I6[4], I6[5], I6[2]]])
+        I = R @ (I - m * (cb @ cb * np.eye(3) - np.outer(cb, cb))) @ R.T
+        c = R @ cb
+        bodies.append((p + c, m * (a + np.cross(al, c) + np.cross(w, np.cross(w, c))), I @ al + np.cross(w, I @ w)))
+        qi += M.NQ[ty]
+        ui += M.DOF[ty]
+    out, terms = np.zeros(spec.nu, L), np.zeros(spec.nu, L)
+    for k, o, ax, first in hinges:
+        for at, f, n in bodies[first:]:
+            x = f if o is None else n + np.cross(at - o, f)
+            y = f if o is None else np.abs(n) + np.abs(np.cross(at - o, f))
+            out[k] += ax @ x
+            terms[k] += np.abs(ax) @ np.abs(y)
+    return out.astype(np.float64), terms.astype(np.float64)
+
+
+def _comp(a, ref):
+    b, terms = ref
+    return float(np.max(np.abs(np.ravel(a) - b) / terms))
+
+
+@pytest.mark.parametrize("m_tip", [1.0, 1e-4, 1e-8])
+@pytest.mark.parametrize("types", [[M.PIN, M.PIN], [M.PIN, M.UNIVERSAL, M.PIN], [M.SLIDER, M.BALL, M.PIN]])
+def test_light_fast_tip(types, m_tip):
+    """M v, the residual and the reactions where the tip's share of the base
+    torque is small although its acceleration is large."""
+    from simbody_amd.matter import MatterBatch
+    spec = _planar(types, [1.0] * (len(types) - 1) + [m_tip])
+    batch = MatterBatch([spec], n_instances=2)
+    q = np.zeros(spec.nq); u = np.zeros(spec.nu); v = np.zeros(spec.nu)
+    qi, ui = spec.offsets()
+    for b, t in enumerate(types):
+        if t == M.BALL:
+            q[qi[b]:qi[b] + 4] = M.Rng(5, b).normal(4)
+            q[qi[b]:qi[b] + 4] /= np.linalg.norm(q[qi[b]:qi[b] + 4])
+        else:
+            q[qi[b]] = 0.3 + 0.2 * b
+    v[0] = 1.0 / 3.0
+    v[-1] = 1.0 / (7.0 * m_tip)
+    u[0] = 0.1
+    o = OracleModel(spec)
+    Q, U, V = (batch.pack([x, x]) for x in (q, u, v))
+    assert _comp(batch.split_u(batch.multiplyByM(Q, V))[1], _residual(spec, q, 0 * u, v)) < 1e-13
+    got = batch.split_u(batch.calcResidualForceIgnoringConstraints(Q, U, udot=V))[1]
+    assert _comp(got, _residual(spec, q, u, v)) < 1e-13
+    # a torque that gives the tip that acceleration
+    f = np.zeros(spec.nu)
+    f[-1] = 0.01
+    F = np.zeros((spec.nb + 1, 6))
+    F[1] = [0.1, 0.2, 0.3, 1.0, 2.0, 3.0]
+    got = np.reshape(batch.split_b(batch.calcMobilizerReactionForces(Q, U, batch.pack([f, f]), batch.pack([F, F])), 6)[1],
+                     (-1, 6))
+    ref = np.reshape(o.reactions(q, u, f, F), (-1, 6))
+    for b in range(1, spec.nb + 1):
+        scale = np.abs(ref[b]).max()
+        assert np.abs(got[b] - ref[b]).max() < 1e-12 * scale, (b, got[b], ref[b])
