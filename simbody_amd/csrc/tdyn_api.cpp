@@ -463,7 +463,7 @@ int tdyn_batch_create(const tdyn_tree_desc* trees, int n_trees, const int32_t* t
         for (int b = 1; b <= nb; ++b) {
             const int ty = trees[0].mobilizer[b-1];
             pack_joint_consts(trees[0], b, prm_j.data() + (size_t)(b-1) * PRM_STRIDE);
-            body_j.push_back(make_int4(ty, B->g_rows, B->tc_rows, 0));
+            body_j.push_back(make_int4(ty, B->g_rows, B->tc_rows, b > 1 ? body_j.back().y : 0));
             B->g_rows += jt_g(ty); B->tc_rows += jt_tc(ty);
         }
         B->jidf = identity_joints(prm_j.data(), nb);

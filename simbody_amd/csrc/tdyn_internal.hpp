@@ -109,7 +109,7 @@ struct DevTables {
     const int* child_idx;    // local body numbers
     const double* prm;       // PRM_STRIDE per global body
     const double* prm_j;     // the same bodies' JC_* constants (batches of one chain)
-    const int4* body_j;      // per global body: mobilizer, first G row, first trig row, -
+    const int4* body_j;      // per global body: mobilizer, first G row, first trig row, its parent's first G row
     const int4* tree_a;      // per tree: nb, nq, nu, body_off
     const int4* tree_b;      // per tree: rec_size, nquat, hand-over base of the chain evaluator, lvl offset
     const double* gravity;   // per tree: 4 doubles

@@ -237,12 +237,6 @@ template <int T> struct Jnt {
         else if constexpr (T == SLIDER) return w;
         else return w + wrel(u);
     }
-    TDJ d3 sub_wrel(const d3& w, const double* u) const {
-        if constexpr (T == PIN) return {w.x, w.y, w.z - u[0]};
-        else if constexpr (T == UNIVERSAL) return {w.x - u[0], w.y - u[1], w.z};
-        else if constexpr (T == SLIDER) return w;
-        else return w - wrel(u);
-    }
     // bias of the angular acceleration, J axes: wp x wrel plus the turning
     // of the hinge columns; wp: the parent's angular velocity in J axes
     TDJ d3 bias_w(const d3& wp, const double* u) const {
@@ -567,20 +561,20 @@ TDJ art zero_art() { art P; for (int k = 0; k < 6; ++k) { P.M.a[k] = 0; P.J.a[k]
 
 // One body of the tip-to-base sweep: P, z (M axes, its children's share in)
 // with the body added, the joint eliminated and the rest taken to the
-// parent's M frame; w: the body's angular velocity in, its parent's out.
-// z already holds minus the applied force.  root: nothing is handed on.
-// VEL: with the velocity terms (else u and w are not read).
+// parent's M frame; w: the body's angular velocity, wpar its parent's (M axes
+// each; not recovered from w, whose rounding would be the parent's where the
+// body turns much faster).  z already holds minus the applied force.  root:
+// nothing is handed on.  VEL: with the velocity terms (else u, w and wpar are
+// not read).
 template <int T, bool IDF, bool TAU, bool VEL = true, class PA>
-TDJ bool in_body(const PA& C, const Jnt<T>& J, const double* u, const double* tau, art& P, wf& z, d3& w, double* g,
-                 bool root) {
+TDJ bool in_body(const PA& C, const Jnt<T>& J, const double* u, const double* tau, art& P, wf& z, const d3& w,
+                 const d3& wpar, double* g, bool root) {
     add_body(C, P);
     if constexpr (VEL) {
         const wf b = gyro(C, w);
         z.w = z.w + b.w; z.v = z.v + b.v;
     }
     to_J<T>(J, P, z);
-    d3 wp;
-    if constexpr (VEL) wp = J.sub_wrel(J.fromB(w), u);
     bool bad;
     if constexpr (T == BALL && TAU) {
         const d3 t = mulT(J.R, d3{tau[0], tau[1], tau[2]});     // given in F
@@ -589,10 +583,9 @@ TDJ bool in_body(const PA& C, const Jnt<T>& J, const double* u, const double* ta
     } else bad = eliminate<T, TAU>(P, z, tau, g);
     if (root) return bad;
     const d3 r = arm<T, IDF>(C, J);
-    if constexpr (VEL) {
-        const d3 wF = J.fromJ(wp);
-        w = fromF<IDF>(C, wF);
-        if constexpr (T != FREE) add_bias<T>(P, z, J.bias_w(wp, u), bias_v<T, IDF>(C, J, w, wF, r, u));
+    if constexpr (VEL && T != FREE) {
+        const d3 wF = toF<IDF>(C, wpar);
+        add_bias<T>(P, z, J.bias_w(J.toJ(wF), u), bias_v<T, IDF>(C, J, wpar, wF, r, u));
     }
     to_F<T, TAU>(J, P, z);
     to_parent<T, IDF, TAU>(C, P, z, r);

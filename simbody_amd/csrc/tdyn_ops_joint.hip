@@ -3,7 +3,7 @@
 //
 // The record-based sweeps (k_op) write and read 0.7-1.6 kB per body between
 // sweeps.  Here a sweep keeps 6 to 12 doubles per body for the next one (G and
-// DI*eps, or the force on the body), the joint angles' sines are formed again,
+// DI*eps, the body's angular velocity, or the force on it), the joint angles' sines are formed again,
 // and rotations are recovered on the way back along the chain; the rest of the
 // traffic is the arguments and the results themselves.
 //
@@ -37,12 +37,13 @@ struct Blk {
     TDJ Blk from(int r) const { return {b + (size_t)r * 64, o}; }
     TDJ TD_GLOBAL double& operator()(int k) const { return *(TD_GLOBAL double*)((TD_GLOBAL char*)(b + k * 64) + o); }
 };
-struct Tab { int y, q, u, g; };
+struct Tab { int y, q, u, g, gp; };        // (gp: the parent's G row)
 
 // What a sweep needs of one body, loaded one body ahead.
-struct In { double q[7], u[6], v[6], f[6], g[12]; };
+struct In { double q[7], u[6], v[6], f[6], g[12], w[3]; };
 
-enum : unsigned { LD_U = 1, LD_V = 2, LD_TAU = 4, LD_F = 8, LD_G = 16, LD_FM = 32 };   // (LD_FM: the force kept, put_force)
+enum : unsigned { LD_U = 1, LD_V = 2, LD_TAU = 4, LD_F = 8, LD_G = 16, LD_FM = 32, LD_W = 64 };
+// (LD_FM: the force kept, put_force; LD_W: the parent's angular velocity, put_w)
 
 template <bool IDF> struct Chain {
     cdptr prm; const int4 *body_a, *body_j;
@@ -50,7 +51,10 @@ template <bool IDF> struct Chain {
     Pk q, u, v, tau, F;         // arguments (v: udot or the vector of M v, J v)
     Pk ou, oq, ob, ob2;         // results
     Blk G;
-    TDJ Tab tab(int b) const { const int4 a = ldi4(body_a, b - 1); return {a.y, a.z, a.w, ldi4(body_j, b - 1).y}; }
+    TDJ Tab tab(int b) const {
+        const int4 a = ldi4(body_a, b - 1), j = ldi4(body_j, b - 1);
+        return {a.y, a.z, a.w, j.y, j.w};
+    }
     TDJ cdptr C(int b) const { return prm + (size_t)(b - 1) * PRM_STRIDE; }
 
     template <int T, unsigned W> TDJ void load(In& x, int b, const Tab& j) const {
@@ -89,6 +93,17 @@ template <bool IDF> struct Chain {
 #pragma unroll
             for (int k = 0; k < 6; ++k) x.g[k] = g(k);
         }
+        if constexpr ((W & LD_W) != 0) {
+            const Blk g = G.from(j.gp);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) x.w[k] = g(k);
+        }
+    }
+    // The angular velocity of body j into its G rows, where the sweep back
+    // reads it before it writes G.
+    TDJ void put_w(const Tab& j, const d3& w) const {
+        const Blk g = G.from(j.g);
+        g(0) = w.x; g(1) = w.y; g(2) = w.z;
     }
     // A force on body j (M axes) into its G rows, and out of them again.
     TDJ void put_force(const Tab& j, const wf& f) const {
@@ -188,10 +203,11 @@ __global__ void __launch_bounds__(64) k_cop(OpArgs a) {
                 constexpr int T = decltype(t)::t;
                 const Jnt<T> J = c.template joint_of<T>(x);
                 w = out_w<T, IDF>(c.C(b), J, w, x.u);
+                c.put_w(j, w);
                 if (hasF) R = out_R<T, IDF>(c.C(b), J, R);
             });
         art P = zero_art(); wf z{zero3<double>(), zero3<double>()};
-        c.template sweep<false, (VEL ? LD_U : 0u) | (TAU ? LD_TAU : 0u) | (FB ? LD_F : 0u)>(
+        c.template sweep<false, (VEL ? LD_U | LD_W : 0u) | (TAU ? LD_TAU : 0u) | (FB ? LD_F : 0u)>(
             [&](auto t, const In& x, int b, const Tab& j) {
                 constexpr int T = decltype(t)::t;
                 const cdptr C = c.C(b);
@@ -202,7 +218,9 @@ __global__ void __launch_bounds__(64) k_cop(OpArgs a) {
                     R = in_R<T, IDF>(C, J, R);
                 }
                 double g[Dim<T>::G];
-                bad |= in_body<T, IDF, TAU, VEL>(C, J, x.u, x.v, P, z, w, g, b == 1);
+                const d3 wpar = {x.w[0], x.w[1], x.w[2]};
+                bad |= in_body<T, IDF, TAU, VEL>(C, J, x.u, x.v, P, z, w, wpar, g, b == 1);
+                w = wpar;
                 const Blk G = c.G.from(j.g);
 #pragma unroll
                 for (int k = 0; k < Dim<T>::G; ++k) G(k) = g[k];

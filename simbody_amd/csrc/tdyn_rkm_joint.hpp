@@ -12,10 +12,16 @@
 // uses only once (stages 1 and 4) never reach memory, and qdot is formed
 // again from the stage's q and u where it is needed.
 //
+// The angular velocities are kept for the sweep back too (three doubles per
+// body, in the rows of its G).  Recovered from the tip's by subtraction they
+// moved 15 % fewer bytes (65,536 x 32: 11.2 ms for 16 steps, 12.6 as it is),
+// but a slow body's carried the rounding of a fast outer one's: udot of two
+// arms with a balanced wheel at 1e7 rad/s was off by 5e-11.
+//
 // What bounds it.  65,536 chains of 32 bodies are one wavefront per SIMD; a
-// step moves 48 kB per instance between the sweeps (half of it G and DI*eps)
-// at 4.4 TB/s, near what a plain copy reaches, and issues half as many vector
-// instructions as the Ground-frame sweeps did: 0.70 ms per step against
+// step moves 57 kB per instance between the sweeps (half of it G and DI*eps)
+// at BW TB/s, near what a plain copy reaches, and issues half as many vector
+// instructions as the Ground-frame sweeps did: 0.79 ms per step against
 // 1.43 ms.  A few chains are bound by the latency of one lane's serial sweeps
 // (one 10-link pendulum: 1.6 against 3.4 ms for 0.1 s at accuracy 1e-8).
 #pragma once
@@ -57,7 +63,7 @@ struct TcL {
 };
 
 // What a sweep needs of one body from memory, loaded a body ahead.
-template <int NQ, int D> struct InB { double q[NQ], u[D], tc[4]; };
+template <int NQ, int D> struct InB { double q[NQ], u[D], tc[4], w[3]; };      // (w: the parent's angular velocity)
 template <int NQ, int D, int G> struct OutB {
     double q[NQ], u[D], tc[4], g[G], yq[NQ], yu[D], f0[D], fq[NQ], fu[D];
 };
@@ -83,6 +89,8 @@ template <class PA, bool IDF, bool HASF, class Rows, class TC> struct Eval {
 #pragma unroll
         for (int k = 0; k < Dim<T>::TC; ++k) tc.put(j.z + k, t[k]);
         w = out_w<T, IDF>(C(b), J, w, u);
+        const Rows G = sc.from(j.y);        // (read on the way back, before G is written there)
+        G(0) = w.x; G(1) = w.y; G(2) = w.z;
         if constexpr (HASF) R = out_R<T, IDF>(C(b), J, R);
     }
     // MODE 0: the state y itself; 1: the first Merson stage y0 + h/3 f0,
@@ -143,6 +151,9 @@ template <class PA, bool IDF, bool HASF, class Rows, class TC> struct Eval {
         }
 #pragma unroll
         for (int k = 0; k < Dim<T>::TC; ++k) x.tc[k] = tc.get(j.z + k);
+        const Rows G = sc.from(j.w);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) x.w[k] = G(k);
     }
     template <int T, class X> TDJ void in_step(const X& x, int b, const int4& j, art& P, wf& z, d3& w, dm& R) const {
         const PA c = C(b);
@@ -156,7 +167,9 @@ template <class PA, bool IDF, bool HASF, class Rows, class TC> struct Eval {
             R = in_R<T, IDF>(c, J, R);
         }
         double g[Dim<T>::G];
-        (void)in_body<T, IDF, false>(c, J, x.u, nullptr, P, z, w, g, b == 1);
+        const d3 wpar = {x.w[0], x.w[1], x.w[2]};
+        (void)in_body<T, IDF, false>(c, J, x.u, nullptr, P, z, w, wpar, g, b == 1);
+        w = wpar;
         const Rows G = sc.from(j.y);
 #pragma unroll
         for (int k = 0; k < Dim<T>::G; ++k) G(k) = g[k];

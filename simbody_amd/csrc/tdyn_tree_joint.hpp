@@ -515,8 +515,8 @@ template <bool IDF, bool HASF> struct GroupJoint {
                 for (int k = 0; k < 6; ++k) u[k] = y.u[bt.z + k];
                 Jnt<FREE> J;
                 J.set(q, d.h + JG_TC);
-                art P0 = P; wf z0 = z; d3 w0 = w;
-                bad |= in_body<FREE, IDF, false>(d.C, J, u, nullptr, P0, z0, w0, g, true);
+                art P0 = P; wf z0 = z;
+                bad |= in_body<FREE, IDF, false>(d.C, J, u, nullptr, P0, z0, w, zero3<double>(), g, true);
                 sto<6>(r, JG_G, g);
                 act = false;
             }

@@ -1,5 +1,5 @@
 """Badly scaled models and states, each quantity on its own scale: a light fast
-distal link.
+distal link; a fast balanced wheel at the end of slow arms.
 
 Tolerances.  A recursion that forms every body's own values from its parent's
 is off by a few roundings of the quantity's own terms: with chains of three
@@ -133,3 +133,62 @@ def test_light_fast_tip(types, m_tip):
     for b in range(1, spec.nb + 1):
         scale = np.abs(ref[b]).max()
         assert np.abs(got[b] - ref[b]).max() < 1e-12 * scale, (b, got[b], ref[b])
+
+
+def _wheel(tree):
+    spec = (_planar([M.PIN, M.PIN, M.PIN, M.PIN], [1.0, 1.0, -0.5, 1.0], parent=[0, 1, 2, 1]) if tree
+            else _planar([M.PIN, M.PIN, M.PIN], [1.0, 1.0, -0.5]))
+    q = np.array([0.4, -0.7, 0.2, 1.1])[:spec.nq]
+    u = np.array([0.9, -1.3, 1e7, 0.5])[:spec.nu]
+    return spec, q, u
+
+
+def _batch(spec, tree):
+    from simbody_amd.matter import MatterBatch
+    if not tree:
+        return MatterBatch([spec], n_instances=3)
+    # another tree beside it: a batch of different trees
+    return MatterBatch([spec, _planar([M.PIN], [1.0])], tree_of=np.array([0, 1, 0], np.int32))
+
+
+def _pack(batch, tree, x):
+    return batch.pack([x, np.zeros(1) if tree else x, x])
+
+
+@pytest.mark.parametrize("tree", [False])
+def test_fast_wheel_accelerations(tree):
+    from simbody_amd.matter import RungeKuttaMerson
+    spec, q, u = _wheel(tree)
+    batch = _batch(spec, tree)
+    Q, U = _pack(batch, tree, q), _pack(batch, tree, u)
+    ref = OracleModel(spec).realize_acceleration(q, u)[0]
+    ud = batch.split_u(batch.realizeAcceleration(Q, U)[0])
+    assert np.abs(ud[2] - ref).max() < 1e-12 * np.abs(ref).max()
+    batch.rollout_begin(Q, U, RungeKuttaMerson(accuracy=1e-6), 0.1)
+    ud = batch.split_u(batch.rollout_derivs()[1])
+    assert np.abs(ud[2] - ref).max() < 1e-12 * np.abs(ref).max()
+    fm, F = np.zeros(spec.nu), np.zeros((spec.nb + 1, 6))
+    if not tree:
+        got = batch.calcAccelerationIgnoringConstraints(Q, U, batch.pack([fm] * 3), batch.pack([F] * 3))[0]
+        ref = OracleModel(spec).forward(q, u, fm, F)[0]
+        assert np.abs(batch.split_u(got)[2] - ref).max() < 1e-12 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("tree", [False])
+@pytest.mark.parametrize("forces", [False, True])
+def test_fast_wheel_rollout(tree, forces):
+    """The arms' own motion over 100 fixed steps: its change against the
+    oracle's, 100 x 5 evaluations of 1e-13 each."""
+    from simbody_amd.matter import RungeKuttaMerson
+    spec, q, u = _wheel(tree)
+    batch = _batch(spec, tree)
+    F = np.zeros((spec.nb + 1, 6))
+    F[2, 5] = F[1, 2] = 0.25
+    fapp = (batch.pack([F, np.zeros((2, 6)) if tree else F, F]) if forces else None)
+    q1, u1, _ = batch.stepTo(_pack(batch, tree, q), _pack(batch, tree, u),
+                             RungeKuttaMerson(accuracy=1e-3, fixed_step=1e-3), 0.1, fapp=fapp)
+    y, _ = OracleModel(spec).integrate(np.concatenate([q, u]), 0.1, 1e-3, fixed_h=1e-3, Fapp=F if forces else None)
+    arms = [0, 1] + ([3] if tree else [])
+    for got, start, ref in ((batch.split_q(q1)[2], q, y[:spec.nq]), (batch.split_u(u1)[2], u, y[spec.nq:])):
+        for k in arms:
+            assert abs(got[k] - ref[k]) < 5e-11 * abs(ref[k] - start[k]), (k, got[k], ref[k])
