@@ -30,12 +30,13 @@
 namespace tdyn {
 namespace joint {
 
-// Record fields of one breadth-first position: w, trig cache and R_GM; G and
-// DI*eps; and what a far parent or child reads: P and z for the parent, A.
+// Record fields of one breadth-first position: the parent's angular velocity
+// in F axes, trig cache and R_GM; G and DI*eps; and what a far parent or child
+// reads: P and z for the parent, A, the position's own angular velocity.
 // Fields lie in pairs, a pair of a block of BW positions side by side, so that
 // a lane moves 16 bytes at a time and a wavefront's lanes share lines (half
 // the memory instructions of single fields, at the same time per rollout).
-enum { JG_W = 0, JG_TC = 3, JG_R = 7, JG_G = 16, JG_DE = 34, JG_PZ = 38, JG_A = 66, JG_NF = 72, JG_PZ_N = 27 };
+enum { JG_W = 0, JG_TC = 3, JG_R = 7, JG_G = 16, JG_DE = 34, JG_PZ = 38, JG_A = 66, JG_WM = 72, JG_NF = 76, JG_PZ_N = 27 };
 static_assert(JG_NF < tgroup::NF, "a request's record room is sized for tgroup::NF");
 
 // A padded generic joint (any mobilizer but Free): X_FM and H_FM in F, the
@@ -138,17 +139,15 @@ template <bool IDF, class PA> TDJ d3 gen_arm(const PA& C, const Gen& J) {
 template <bool IDF, class PA> TDJ d3 gen_bias_v(const PA& C, const Gen& J, const d3& w, const d3& wF, const d3& r, const double* u) {
     return toF<IDF>(C, centripetal(w, r)) + 2.0*cross(wF, J.vrel(u));
 }
-// As in_body; g: G (18) and DI*eps (3).  ahead: called when C, u and w are
-// in use no more.
+// As in_body; wF: the parent's angular velocity in F axes; g: G (18) and DI*eps
+// (3).  ahead: called when C and u are in use no more.
 template <bool IDF, class PA, class Fn>
-TDJ bool gen_in(const PA& C, const Gen& J, const double* u, art& P, wf& z, d3& w, double* g, Fn&& ahead) {
+TDJ bool gen_in(const PA& C, const Gen& J, const double* u, art& P, wf& z, const d3& wF, double* g, Fn&& ahead) {
     add_body(C, P);
-    const wf b = gyro(C, w);
+    const wf b = gyro(C, mulT(J.R, wF + J.wrel(u)));
     // the body's transfer to its parent: bias accelerations (F), arm
-    const d3 wF = mul(J.R, w) - J.wrel(u);
-    w = fromF<IDF>(C, wF);
     const d3 r = gen_arm<IDF>(C, J);
-    const d3 aw = J.bias_w(wF, u), av = gen_bias_v<IDF>(C, J, w, wF, r, u);
+    const d3 aw = J.bias_w(wF, u), av = gen_bias_v<IDF>(C, J, fromF<IDF>(C, wF), wF, r, u);
     dm Rc;
     if constexpr (!IDF) for (int i = 0; i < 9; ++i) Rc.a[i] = C[JC_R + i];
     ahead();
@@ -208,14 +207,12 @@ TDJ bool gen_in(const PA& C, const Gen& J, const double* u, art& P, wf& z, d3& w
     z.w = z.w + cross(r, z.v);
     return !(det > 0.0);
 }
-// As out_body, from the body's own angular velocity wm (M axes).
+// As out_body; wF as above.
 template <bool IDF, class PA>
-TDJ void gen_out(const PA& C, const Gen& J, const double* u, const double* g, wf& A, const d3& wm, double* ud) {
+TDJ void gen_out(const PA& C, const Gen& J, const double* u, const double* g, wf& A, const d3& wF, double* ud) {
     const d3 r = gen_arm<IDF>(C, J);
-    const d3 wF = mul(J.R, wm) - J.wrel(u);
-    const d3 w = fromF<IDF>(C, wF);
     wf a;
-    a.v = toF<IDF>(C, A.v + cross(A.w, r)) + gen_bias_v<IDF>(C, J, w, wF, r, u);
+    a.v = toF<IDF>(C, A.v + cross(A.w, r)) + gen_bias_v<IDF>(C, J, fromF<IDF>(C, wF), wF, r, u);
     a.w = toF<IDF>(C, A.w) + J.bias_w(wF, u);
 #pragma unroll
     for (int j = 0; j < 3; ++j)
@@ -367,10 +364,12 @@ template <bool IDF, bool HASF> struct GroupJoint {
         else { qd[0] = u[0]; qd[1] = u[1]; qd[2] = u[2]; qd[3] = 0.0; }
     }
 
-    // Angular velocity, trig cache (and rotation) of position j into the record
-    // and for its children.
-    TDJ void pass_on(int j, const int4& e, double* r, const d3& w, const double* tc, const dm& R) const {
-        double x[16] = {w.x, w.y, w.z, tc[0], tc[1], tc[2], tc[3]};
+    // The parent's angular velocity in F axes (wF), trig cache (and rotation) of
+    // position j into the record, its own angular velocity (and rotation) to its
+    // children.  (wF is kept rather than w: recovered from w, a slow parent's
+    // would carry the rounding of a fast body's.)
+    TDJ void pass_on(int j, const int4& e, double* r, const d3& wF, const d3& w, const double* tc, const dm& R) const {
+        double x[16] = {wF.x, wF.y, wF.z, tc[0], tc[1], tc[2], tc[3]};
 #pragma unroll
         for (int k = 0; k < 9; ++k) x[7 + k] = HASF ? R.a[k] : 0.0;
         sto<HASF ? 16 : 8>(r, JG_W, x);
@@ -379,28 +378,40 @@ template <bool IDF, bool HASF> struct GroupJoint {
             if constexpr (HASF)
 #pragma unroll
                 for (int k = 0; k < 9; ++k) fr(3 + k, j) = R.a[k];
+            // (a position's children follow each other)
+            if (!near(e.z + e.w - 1, j)) {
+                const double y[3] = {w.x, w.y, w.z};
+                sto<3>(r, JG_WM, y);
+            }
         }
     }
     TDJ void of_parent(int j, const int4& e, d3& w, dm& R) const {
         w = zero3<double>(); R = ident<double>();
         if (e.y < 0) return;
-        double x[16];
+        double x[4], y[10];
         if (near(j, e.y)) {
 #pragma unroll
-            for (int k = 0; k < 3 + kR; ++k) x[k < 3 ? k : k + 4] = fr(k, e.y);
+            for (int k = 0; k < 3; ++k) x[k] = fr(k, e.y);
+#pragma unroll
+            for (int k = 0; k < kR; ++k) y[1 + k] = fr(3 + k, e.y);
         } else {
-            ld<HASF ? 16 : 4>(rec(e.y), JG_W, x);
+            const double* r = rec(e.y);
+            ld<3>(r, JG_WM, x);
+            if constexpr (HASF) ld<10>(r, JG_R - 1, y);
         }
         w = {x[0], x[1], x[2]};
         if constexpr (HASF)
 #pragma unroll
-            for (int k = 0; k < 9; ++k) R.a[k] = x[7 + k];
+            for (int k = 0; k < 9; ++k) R.a[k] = y[1 + k];
     }
-    // X and w of the generic position j at (q, u) and its trig cache.
-    template <class C> TDJ void turn(int ty, const C& K, const double* q, const double* u, double* tc, d3& w, dm& R) const {
+    // X and w of the generic position j at (q, u) and its trig cache (w, R: the
+    // parent's in, the position's out).
+    template <class C>
+    TDJ void turn(int ty, const C& K, const double* q, const double* u, double* tc, d3& wF, d3& w, dm& R) const {
         Gen J;
         Gen::trig(ty, q, tc); J.set(ty, q, tc, K[JC_PITCH]);
-        w = mulT(J.R, toF<IDF>(K, w) + J.wrel(u));
+        wF = toF<IDF>(K, w);
+        w = mulT(J.R, wF + J.wrel(u));
         if constexpr (HASF) {
             if constexpr (!IDF) { dm B; for (int k = 0; k < 9; ++k) B.a[k] = K[JC_R + k]; R = mul(R, B); }
             R = mul(R, J.R);
@@ -452,20 +463,21 @@ template <bool IDF, bool HASF> struct GroupJoint {
                 for (int k = 0; k < 6; ++k) u[k] = y.u[bt.z + k];
                 double tc[4];
                 turn_free(d.C, q, u, tc, w, R);
-                pass_on(j, e, r, w, tc, R);
+                pass_on(j, e, r, zero3<double>(), w, tc, R);
                 act = false;
             }
             mask_u(bt.x, d.u);
             double tc[4];
-            turn(bt.x, d.C, d.q, d.u, tc, w, R);
+            d3 wF;
+            turn(bt.x, d.C, d.q, d.u, tc, wF, w, R);
             ahead();
-            if (act) pass_on(j, e, r, w, tc, R);
+            if (act) pass_on(j, e, r, wF, w, tc, R);
         });
     }
 
     // The inward sweep at y; true when some body's D was not positive definite.
     __device__ __forceinline__ bool inward(const QU& y) const {
-        struct D { double C[JC_STRIDE], q[4], u[3], h[16], f[6]; };   // h: w, trig cache, R
+        struct D { double C[JC_STRIDE], q[4], u[3], h[16], f[6]; };   // h: wF, trig cache, R
         bool bad = false;
         inward_steps<D>([&](D& d, int j, const int4& bt) {
             double* r = rec(j);
@@ -498,7 +510,7 @@ template <bool IDF, bool HASF> struct GroupJoint {
                 z.v = z.v + d3{q[24], q[25], q[26]};
             }
             grp_sync();
-            d3 w = {d.h[0], d.h[1], d.h[2]};
+            const d3 wF = {d.h[0], d.h[1], d.h[2]};
             if constexpr (HASF) {
                 dm R;
 #pragma unroll
@@ -516,7 +528,8 @@ template <bool IDF, bool HASF> struct GroupJoint {
                 Jnt<FREE> J;
                 J.set(q, d.h + JG_TC);
                 art P0 = P; wf z0 = z;
-                bad |= in_body<FREE, IDF, false>(d.C, J, u, nullptr, P0, z0, w, zero3<double>(), g, true);
+                const d3 w = out_w<FREE, IDF>(d.C, J, wF, u);
+                bad |= in_body<FREE, IDF, false>(d.C, J, u, nullptr, P0, z0, w, wF, g, true);
                 sto<6>(r, JG_G, g);
                 act = false;
             }
@@ -524,7 +537,7 @@ template <bool IDF, bool HASF> struct GroupJoint {
             Gen J;
             J.set(bt.x, d.q, d.h + JG_TC, d.C[JC_PITCH]);
             double g[21];
-            bad |= gen_in<IDF>(d.C, J, d.u, P, z, w, g, ahead) && act;
+            bad |= gen_in<IDF>(d.C, J, d.u, P, z, wF, g, ahead) && act;
             if (act) {
                 sto<21>(r, JG_G, g);
                 if (e.y >= 0) {
@@ -613,7 +626,7 @@ template <bool IDF, bool HASF> struct GroupJoint {
                     d3 w0 = zero3<double>(); dm R0 = ident<double>();
                     double tc[4];
                     turn_free(d.C, x, x + 7, tc, w0, R0);
-                    pass_on(j, e, r, w0, tc, R0);
+                    pass_on(j, e, r, zero3<double>(), w0, tc, R0);
                 } else {
                     if (f.q)
 #pragma unroll
@@ -628,8 +641,7 @@ template <bool IDF, bool HASF> struct GroupJoint {
             J.set(bt.x, d.q, d.h + JG_TC, d.C[JC_PITCH]);
             double k1[7];
             qdot(bt.x, d.q, d.u, k1);
-            const d3 wm = {d.h[0], d.h[1], d.h[2]};
-            gen_out<IDF>(d.C, J, d.u, d.g, A, wm, k1 + 4);
+            gen_out<IDF>(d.C, J, d.u, d.g, A, d3{d.h[0], d.h[1], d.h[2]}, k1 + 4);
             const int nqb = mob_nq(bt.x), nub = J.d;
             if constexpr (NEXT) {
                 double x[7], er[7];
@@ -656,10 +668,10 @@ template <bool IDF, bool HASF> struct GroupJoint {
                 }
                 mask_u(bt.x, x + 4);
                 double tc[4];
-                d3 w; dm R;
+                d3 wF, w; dm R;
                 of_parent(j, e, w, R);
-                turn(bt.x, K, x, x + 4, tc, w, R);
-                if (act) pass_on(j, e, r, w, tc, R);
+                turn(bt.x, K, x, x + 4, tc, wF, w, R);
+                if (act) pass_on(j, e, r, wF, w, tc, R);
             } else {
                 ahead();
                 if (act) {

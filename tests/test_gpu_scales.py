@@ -155,7 +155,7 @@ def _pack(batch, tree, x):
     return batch.pack([x, np.zeros(1) if tree else x, x])
 
 
-@pytest.mark.parametrize("tree", [False])
+@pytest.mark.parametrize("tree", [False, True])
 def test_fast_wheel_accelerations(tree):
     from simbody_amd.matter import RungeKuttaMerson
     spec, q, u = _wheel(tree)
@@ -174,7 +174,7 @@ def test_fast_wheel_accelerations(tree):
         assert np.abs(batch.split_u(got)[2] - ref).max() < 1e-12 * np.abs(ref).max()
 
 
-@pytest.mark.parametrize("tree", [False])
+@pytest.mark.parametrize("tree", [False, True])
 @pytest.mark.parametrize("forces", [False, True])
 def test_fast_wheel_rollout(tree, forces):
     """The arms' own motion over 100 fixed steps: its change against the
