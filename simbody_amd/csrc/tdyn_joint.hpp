@@ -136,17 +136,23 @@ TDJ void shift_universal(art& P, const d3& r) {
 }
 
 // sin and cos for |x| < 2^20, the library's beyond.  x - k pi/2 in three parts
-// (Cody and Waite; the first is exact in one fused multiply-add), then
-// polynomials in r^2 through the Chebyshev nodes of [0, (pi/4)^2] (largest
-// error 2e-17) and the rest of r to first order: 40 instructions where the
-// library's small-argument path takes 130, under 1 ulp as that is.  One angle
-// per body and derivative made it a sixth of a chain derivative.
+// (Cody and Waite): the first is exact in one fused multiply-add, the second a
+// product with its error, subtracted with the error of the difference (next to
+// a multiple of pi/2 the difference is as small as the product's rounding
+// would be), so that r + lo is the remainder to 2^-100.  Then polynomials in
+// r^2 through the Chebyshev nodes of [0, (pi/4)^2] (largest error 2e-17) and lo
+// to first order: 46 instructions where the library's small-argument path takes
+// 130, under 1 ulp as that is.  One angle per body and derivative made it a
+// sixth of a chain derivative.
 TDJ bool big_angle(double x) { return !(fabs(x) < 1048576.0); }
 TDJ void sincos_small(double x, double* sp, double* cp) {
+#pragma clang fp contract(off)
     const double k = rint(x * 0.6366197723675814);
     const double t = fma(-k, 1.5707963267948966, x);
-    const double r = fma(-k, 6.123233995736766e-17, t);
-    const double lo = fma(-k, -1.4973849048591698e-33, fma(-k, 6.123233995736766e-17, t - r));
+    const double p = k * 6.123233995736766e-17, pe = fma(k, 6.123233995736766e-17, -p);
+    const double r = t - p, rb = r - t;
+    const double re = (t - (r - rb)) - (p + rb);
+    const double lo = fma(-k, -1.4973849048591698e-33, re - pe);
     const double z = r*r;
     const double ps = fma(z, fma(z, fma(z, fma(z, fma(z, 1.591810123027412e-10, -2.5051131455427946e-08),
                                                 2.755731610068303e-06), -0.0001984126983675497),

@@ -1,5 +1,6 @@
 """Badly scaled models and states, each quantity on its own scale: a light fast
-distal link; a fast balanced wheel at the end of slow arms.
+distal link; a fast balanced wheel at the end of slow arms; angles next to
+the zeros of their cosine.
 
 Tolerances.  A recursion that forms every body's own values from its parent's
 is off by a few roundings of the quantity's own terms: with chains of three
@@ -192,3 +193,20 @@ def test_fast_wheel_rollout(tree, forces):
     for got, start, ref in ((batch.split_q(q1)[2], q, y[:spec.nq]), (batch.split_u(u1)[2], u, y[spec.nq:])):
         for k in arms:
             assert abs(got[k] - ref[k]) < 5e-11 * abs(ref[k] - start[k]), (k, got[k], ref[k])
+
+
+def test_cosine_next_to_its_zeros():
+    """A pendulum's udot is a constant times the cosine of its angle where
+    gravity is along the link's normal at zero: relative accuracy at and
+    beside multiples of pi/2 up to 2^20 (three roundings of the result)."""
+    from simbody_amd.matter import MatterBatch
+    spec = _planar([M.PIN], [1.0])
+    k = np.unique(np.concatenate([np.arange(1, 400, 2), np.geomspace(401, 667000, 3000).astype(np.int64) | 1]))
+    x0 = (k.astype(np.longdouble) * (np.longdouble("3.14159265358979323846264338327950288") / 2)).astype(np.float64)
+    x = np.concatenate([x0, np.nextafter(x0, 0), np.nextafter(x0, np.inf), -x0, [0.0]])
+    batch = MatterBatch([spec], n_instances=len(x))
+    ud = batch.realizeAcceleration(batch.to_device(x), batch.to_device(np.zeros(len(x))))[0].cpu().numpy()
+    c = np.cos(x.astype(np.longdouble))
+    err = np.abs(ud / ud[-1] - c) / np.abs(c)
+    worst = int(np.argmax(err))
+    assert err[worst] < 1e-15, (x[worst], float(err[worst]))
