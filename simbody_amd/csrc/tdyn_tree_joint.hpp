@@ -97,7 +97,8 @@ struct Gen {
         c1 = ball ? 1.0 : univ ? R.a[4] : 0.0; d1 = univ ? R.a[7] : 0.0;
         h2 = {0.0, 0.0, ball ? 1.0 : 0.0};
         hv1 = hv2 = zero3<double>();
-        p = {v0*q[0], 0.0, v0z*q[0]};
+        // (selected, not multiplied: a Weld's q[0] is another body's)
+        p = {v0 != 0.0 ? q[0] : 0.0, 0.0, v0z != 0.0 ? v0z*q[0] : 0.0};
         if (ty == SLIDER || ty == WELD) { R = ident<double>(); }
         if (tr) {
             if (ty == TRANSLATION) { hv1.y = 1.0; hv2.z = 1.0; p.y = q[1]; p.z = q[2]; }

@@ -1,6 +1,6 @@
 """Badly scaled models and states, each quantity on its own scale: a light fast
 distal link; a fast balanced wheel at the end of slow arms; angles next to
-the zeros of their cosine.
+the zeros of their cosine; a branch that is not a number beside one that is.
 
 Tolerances.  A recursion that forms every body's own values from its parent's
 is off by a few roundings of the quantity's own terms: with chains of three
@@ -210,3 +210,16 @@ def test_cosine_next_to_its_zeros():
     err = np.abs(ud / ud[-1] - c) / np.abs(c)
     worst = int(np.argmax(err))
     assert err[worst] < 1e-15, (x[worst], float(err[worst]))
+
+
+def test_branch_beside_one_that_is_not_a_number():
+    """Base branches do not touch each other: a Weld of one reads nothing of
+    the other's coordinates."""
+    from simbody_amd.matter import MatterBatch
+    spec = _planar([M.PIN, M.WELD, M.PIN], [1.0, 1.0, 1.0], parent=[0, 1, 0])
+    one = _planar([M.PIN], [1.0])
+    batch = MatterBatch([spec, one], tree_of=np.array([0, 1, 0], np.int32))
+    q = [np.array([0.3, np.nan]), np.zeros(1), np.array([0.3, 0.2])]
+    u = [np.array([0.1, 0.2]), np.zeros(1), np.array([0.1, 0.2])]
+    ud = batch.split_u(batch.realizeAcceleration(batch.pack(q), batch.pack(u))[0])
+    assert ud[0][0] == ud[2][0] and np.isnan(ud[0][1])
