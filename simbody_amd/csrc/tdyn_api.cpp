@@ -168,6 +168,28 @@ int make_rkm_cfg(const tdyn_integrator_cfg* cfg, RkmCfg& c, int& precision) {
     return TDYN_OK;
 }
 
+// Estimates of realizeAcceleration of one tree in n instances, us, from runs of
+// 4 to 128 bodies (chains from two bases, 4 and 8 arms, binary trees; one type of
+// joint or mixed; 1 to 4,096 instances).  Level-parallel with 16 lanes: by the
+// steps of a sweep, which are cut where a position's parent is in the step
+// (within 8 %).  One lane each: by body, with the records within the L2 caches
+// (of 8 XCDs, 4 MB each) or beyond (within 7 %).  A chain of 128 bodies from two
+// bases, one instance: 806 us level-parallel, 731 one lane; 48 bodies in 4 arms:
+// 87 and 269.
+double group_op_us(const int4* bfs, int nb, int64_t waves, bool identity) {
+    int steps = 0;
+    for (int s = 0; s < nb; ++steps) s = std::min({s + 16, bfs[s].z, nb});
+    return 7.0 + (identity ? 6.3 : 7.2) * steps + 0.02 * (double)waves;
+}
+double one_lane_op_us(const int4* body_a, int nb, int64_t n, int64_t rec) {
+    double us = 0.0;
+    for (int b = 0; b < nb; ++b) {
+        const int ty = body_a[b].y;
+        us += ty == TDYN_PIN || ty == TDYN_SLIDER ? 5.0 : ty == TDYN_UNIVERSAL ? 6.2 : ty == TDYN_BALL ? 6.7 : 7.3;
+    }
+    const int64_t lanes_per_xcd = std::min<int64_t>(n, ((n + 63) / 64 + 7) / 8 * 64);
+    return lanes_per_xcd * 8 * rec > (4 << 20) ? 5.0 + 1.22 * us : 5.0 + us;
+}
 // Wavefront plan of the level-parallel tree evaluator for the next rollout
 // (returns 0 and leaves the plan empty for the one-lane streaming
 // evaluator).  Lanes per instance: G, the tree_lanes setting, or automatic:
@@ -187,7 +209,13 @@ int make_rkm_cfg(const tdyn_integrator_cfg* cfg, RkmCfg& c, int& precision) {
 // by size; body-steps/s): 4, 8, 16, 32, 64 lanes for every instance 0.56,
 // 1.06, 1.32, 1.27, 0.95 x 1e8; per instance its widest level in [16, 32]
 // 1.31e8.
-int make_tree_plan(tdyn_batch* b, int tree_lanes, tdyn_batch::Plan& P) {
+// op: the operators' plan (one derivative of every instance).  Where instances
+// wait for lanes there, lanes that mostly idle are given up: the lanes are halved
+// while the instances' steps together grow by an eighth at most (16,384
+// different chains of 16 bodies: 436 us with 16 lanes, 160 with 4, one lane each
+// 325; of 128 bodies 3,457, 1,222 and 2,805), and an instance has lanes_max then
+// only where these halve its steps and it is twice the mean load.
+int make_tree_plan(tdyn_batch* b, int tree_lanes, tdyn_batch::Plan& P, bool op = false) {
     const int L = b->n_inst;
     const int64_t resident = std::max(1, tree_group_resident_waves());
     int gq = tree_lanes > 1 ? tree_lanes : b->lanes_min;
@@ -195,12 +223,18 @@ int make_tree_plan(tdyn_batch* b, int tree_lanes, tdyn_batch::Plan& P) {
         gq = 4;
         while (gq < 16 && (int64_t)L * 2 * gq <= 4 * 64 * resident) gq *= 2;
     }
-    const int gbig = tree_lanes > 1 ? gq : std::max(gq, b->lanes_max);
     auto steps = [&](int l, int G) {
         int64_t c = 0;
         for (int w : b->h_tree_lw[b->h_lane_tree[l]]) c += (w + G - 1) / G;
         return c;
     };
+    bool fewer = false;
+    for (; op && gq > 4 && (int64_t)L * gq > 64 * resident; gq /= 2, fewer = true) {
+        int64_t now = 0, half = 0;
+        for (int l = 0; l < L; ++l) { now += steps(l, gq); half += steps(l, gq / 2); }
+        if (8 * half > 9 * now) break;
+    }
+    const int gbig = tree_lanes > 1 ? gq : std::max(gq, b->lanes_max);
     std::vector<int64_t> cost(L);
     int64_t total = 0;
     for (int l = 0; l < L; ++l) { cost[l] = steps(l, gq); total += cost[l]; }
@@ -210,7 +244,11 @@ int make_tree_plan(tdyn_batch* b, int tree_lanes, tdyn_batch::Plan& P) {
     // the mean load of one group slot of the resident wavefronts
     const double mean_load = (double)total / (double)(resident * (64 / gq));
     std::vector<int> big, rest;
-    for (int l : ord) ((gbig > gq && cost[l] > mean_load) ? big : rest).push_back(l);
+    auto is_big = [&](int l) {
+        if (gbig <= gq || !(cost[l] > mean_load)) return false;
+        return !fewer || (cost[l] > 2 * mean_load && 2 * steps(l, gbig) <= cost[l]);
+    };
+    for (int l : ord) (is_big(l) ? big : rest).push_back(l);
     std::vector<int4> plan; std::vector<int> idx;
     for (size_t k = 0; k < big.size(); k += 64 / gbig) {
         const int cnt = (int)std::min(big.size() - k, (size_t)(64 / gbig));
@@ -502,15 +540,19 @@ int tdyn_batch_create(const tdyn_tree_desc* trees, int n_trees, const int32_t* t
     B->h_lane_tree = lane_tree;
     {
     }
-    // Forward dynamics of such trees runs level-parallel, one tree in many
-    // instances only where each has its group of 16 lanes at once: 1,024 x 48
+    // Forward dynamics of such trees runs level-parallel.  One tree in many
+    // instances only where each has its group of 16 lanes at once (1,024 x 48
     // bodies 369 -> 74 us, 4,096 x 48 370 -> 99; with more instances the
-    // one-lane kernel fills the device by itself (16,384 x 16 142 us, 234
-    // level-parallel; 65,536 x 48 1,373, 1,482).  Different trees, whose lanes
-    // walk apart in the one-lane kernel, always: 16,384 of 8 to 128 bodies
-    // 3,230 -> 371 us, 65,536 of 8 to 16 1,062 -> 303.
+    // one-lane kernel fills the device by itself: 16,384 x 16 142 us, 234
+    // level-parallel; 65,536 x 48 1,373, 1,482) and the tree is wide enough for
+    // its steps (group_op_us, one_lane_op_us).  Different trees, whose lanes walk
+    // apart in the one-lane kernel, always: 16,384 of 8 to 128 bodies 3,230 ->
+    // 371 us, 65,536 of 8 to 16 1,062 -> 303.
+    const int64_t group_waves = ((int64_t)n_instances + 3) / 4;
     grp_ok = grp_ok && !B->is_chain && !B->extended() &&
-             (!B->uniform || (int64_t)n_instances * 16 <= (int64_t)64 * std::max(1, tree_group_resident_waves()));
+             (!B->uniform || (group_waves <= std::max(1, tree_group_resident_waves()) &&
+                              group_op_us(bfs.data(), trees[0].nb, group_waves, B->idf_all) <
+                              one_lane_op_us(B->h_body_a.data(), trees[0].nb, n_instances, (int64_t)B->max_rec + 24)));
     size_t n_scratch = (size_t)std::max({B->max_rec + 24, B->stream_ok ? B->stream_stride : 0,
                                          B->stream_ok || grp_ok ? B->group_stride : 0}) * n_instances;
     // (the joint-frame operators keep G rows in blocks of 64 lanes)
@@ -545,7 +587,7 @@ int tdyn_batch_create(const tdyn_tree_desc* trees, int n_trees, const int32_t* t
     // operators allocate nothing (they may be captured)
     if (grp_ok) {
         int rc = ensure_bfs_consts(B, false);
-        if (!rc) rc = make_tree_plan(B, 0, B->op_plan);
+        if (!rc) rc = make_tree_plan(B, 0, B->op_plan, true);
         if (rc) { delete B; return rc; }
     }
     *out = B;
