@@ -46,7 +46,7 @@ enum : unsigned { LD_U = 1, LD_V = 2, LD_TAU = 4, LD_F = 8, LD_G = 16, LD_FM = 3
 // (LD_FM: the force kept, put_force; LD_W: the parent's angular velocity, put_w)
 
 template <bool IDF> struct Chain {
-    cdptr prm; const int4 *body_a, *body_j;
+    cdptr prm, prm_g; const int4 *body_a, *body_j;
     int nb, nq, nu;
     Pk q, u, v, tau, F;         // arguments (v: udot or the vector of M v, J v)
     Pk ou, oq, ob, ob2;         // results
@@ -160,6 +160,23 @@ template <bool IDF> struct Chain {
         else { dm B; for (int i = 0; i < 9; ++i) B.a[i] = c[JC_RB + i]; return mul(R, B); }
     }
     static TDJ d3 Bo(const cdptr& c) { return {c[JC_B], c[JC_B + 1], c[JC_B + 2]}; }
+    // Body b's own mass, first moment and inertia about Bo, M axes: from the
+    // constants about Bo, as those about M have lost what the distance of the
+    // joint adds (a last body of radius 0.001, its joint 3 away: 1e-10 of its
+    // inertia).
+    struct Own { double m; d3 mc; sym I; };
+    TDJ Own own(int b) const {
+        const cdptr g = prm_g + (size_t)(b - 1) * PRM_STRIDE, c = C(b);
+        const double m = g[PRM_MASS];
+        Own o{m, m*d3{g[PRM_COM], g[PRM_COM + 1], g[PRM_COM + 2]}, {}};
+#pragma unroll
+        for (int k = 0; k < 6; ++k) o.I.a[k] = m*g[PRM_G + k];
+        if constexpr (!IDF) {
+            dm B; for (int i = 0; i < 9; ++i) B.a[i] = c[JC_RB + i];
+            o.mc = mul(B, o.mc); o.I = rot(B, o.I);
+        }
+        return o;
+    }
     static TDJ wf force_M(const cdptr& c, const dm& R, const double* f) {
         const d3 fm = mulT(R, d3{f[3], f[4], f[5]});
         return {mulT(R, d3{f[0], f[1], f[2]}) + cross(Bo(c), fm), fm};
@@ -175,6 +192,53 @@ template <bool IDF> struct Chain {
     static TDJ void put0(const Pk& o, int n) { for (int k = 0; k < n; ++k) o(k) = 0.0; }
 };
 
+// P - P H D^-1 H^T P about a point at b from M (M axes).
+template <int T> TDJ void hinge_out(art& P, const Jnt<T>& J, const d3& b) {
+    constexpr int N = Dim<T>::D;
+    wf H[N], U[N];
+    if constexpr (T == SLIDER) H[0] = {zero3<double>(), {1.0, 0.0, 0.0}};
+    else {
+        if constexpr (T == PIN) H[0].w = {0.0, 0.0, 1.0};
+        else if constexpr (T == UNIVERSAL) { H[0].w = J.toB({1.0, 0.0, 0.0}); H[1].w = J.toB({0.0, 1.0, 0.0}); }
+        else { H[0].w = {1.0, 0.0, 0.0}; H[1].w = {0.0, 1.0, 0.0}; H[2].w = {0.0, 0.0, 1.0}; }
+        for (int k = 0; k < N; ++k) H[k].v = cross(H[k].w, b);
+    }
+    double D[N][N], DI[N][N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) U[k] = {mulsym(P.J, H[k].w) + mulF(P.F, H[k].v), mulFt(P.F, H[k].w) + mulsym(P.M, H[k].v)};
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int k = 0; k < N; ++k) D[i][k] = dot(H[i].w, U[k].w) + dot(H[i].v, U[k].v);
+    if constexpr (N == 1) DI[0][0] = 1.0 / D[0][0];
+    else if constexpr (N == 2) {
+        const double o = 1.0 / (D[0][0]*D[1][1] - D[0][1]*D[1][0]);
+        DI[0][0] = o*D[1][1]; DI[1][1] = o*D[0][0]; DI[0][1] = DI[1][0] = -(o*D[0][1]);
+    } else {
+        const double c00 = D[1][1]*D[2][2] - D[1][2]*D[1][2], c01 = D[1][2]*D[0][2] - D[0][1]*D[2][2],
+                     c02 = D[0][1]*D[1][2] - D[1][1]*D[0][2], o = 1.0 / (D[0][0]*c00 + D[0][1]*c01 + D[0][2]*c02);
+        DI[0][0] = o*c00; DI[0][1] = DI[1][0] = o*c01; DI[0][2] = DI[2][0] = o*c02;
+        DI[1][1] = o*(D[0][0]*D[2][2] - D[0][2]*D[0][2]);
+        DI[1][2] = DI[2][1] = o*(D[0][1]*D[0][2] - D[0][0]*D[1][2]);
+        DI[2][2] = o*(D[0][0]*D[1][1] - D[0][1]*D[0][1]);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        wf G{zero3<double>(), zero3<double>()};
+#pragma unroll
+        for (int k = 0; k < N; ++k) { G.w = G.w + DI[i][k]*U[k].w; G.v = G.v + DI[i][k]*U[k].v; }
+        const double gw[3] = {G.w.x, G.w.y, G.w.z}, gv[3] = {G.v.x, G.v.y, G.v.z};
+        const double uw[3] = {U[i].w.x, U[i].w.y, U[i].w.z}, uv[3] = {U[i].v.x, U[i].v.y, U[i].v.z};
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                P.F[3*r + c] -= gw[r]*uv[c];
+                if (c >= r) { P.J.a[sidx(r, c)] -= gw[r]*uw[c]; P.M.a[sidx(r, c)] -= gv[r]*uv[c]; }
+            }
+    }
+}
+
 template <int OP, bool IDF>
 __global__ void __launch_bounds__(64) k_cop(OpArgs a) {
     const int lane = blockIdx.x * 64 + threadIdx.x;
@@ -182,7 +246,7 @@ __global__ void __launch_bounds__(64) k_cop(OpArgs a) {
     Chain<IDF> c;
     const int4 ta = ldi4(a.T.tree_a, 0);
     c.nb = ta.x; c.nq = ta.y; c.nu = ta.z;
-    c.prm = cptr(a.T.prm_j); c.body_a = a.T.body_a; c.body_j = a.T.body_j;
+    c.prm = cptr(a.T.prm_j); c.prm_g = cptr(a.T.prm); c.body_a = a.T.body_a; c.body_j = a.T.body_j;
     const size_t first = (size_t)blockIdx.x * 64;
     c.q = packed(a.q, first, c.nq); c.u = packed(a.u, first, c.nu);
     c.v = packed(a.udot_in, first, c.nu); c.tau = packed(a.fmob, first, c.nu);
@@ -385,9 +449,8 @@ __global__ void __launch_bounds__(64) k_cop(OpArgs a) {
         } else if constexpr (OP == OP_ABI) {
             const Pk oP = packed(a.out_abi, first, 21*(c.nb + 1)), oPP = packed(a.out_abi2, first, 21*(c.nb + 1));
             art P = zero_art(); wf z{zero3<double>(), zero3<double>()};
-            // at Bo in Ground, blocks M, J (xx yy zz xy xz yz), F
-            auto put = [&](const Pk& o, art X, const dm& Rg, const d3& b) {
-                shift(X, -b);
+            // blocks M, J (xx yy zz xy xz yz), F in Ground
+            auto put = [&](const Pk& o, art X, const dm& Rg) {
                 X.M = rot(Rg, X.M); X.J = rot(Rg, X.J); rot(Rg, X.F);
 #pragma unroll
                 for (int k = 0; k < 6; ++k) { o(k) = X.M.a[k]; o(6 + k) = X.J.a[k]; }
@@ -398,23 +461,26 @@ __global__ void __launch_bounds__(64) k_cop(OpArgs a) {
                 constexpr int T = decltype(t)::t;
                 const cdptr C = c.C(b);
                 const Jnt<T> J = c.template joint_of<T>(x);
-                art Q = P;
-                add_body(C, Q);
-                put(oP.from(21*b), Q, R, c.Bo(C));
+                {
+                    // about Bo: the children's share moved there, and the body's own
+                    const auto o = c.own(b);
+                    art Q = P;
+                    shift(Q, -c.Bo(C));
+                    Q.M.a[0] += o.m; Q.M.a[1] += o.m; Q.M.a[2] += o.m;
+#pragma unroll
+                    for (int k = 0; k < 6; ++k) Q.J.a[k] += o.I.a[k];
+                    Q.F[1] -= o.mc.z; Q.F[2] += o.mc.y; Q.F[3] += o.mc.z; Q.F[5] -= o.mc.x; Q.F[6] -= o.mc.y; Q.F[7] += o.mc.x;
+                    put(oP.from(21*b), Q, R);
+                    if (oPP) {
+                        if constexpr (T == FREE) Q = zero_art(); else hinge_out<T>(Q, J, c.Bo(C));
+                        put(oPP.from(21*b), Q, R);
+                    }
+                }
                 double g[Dim<T>::G];
-                // P+ in J axes: the body's own elimination, left before the transfer
-                art X = Q; wf y = z;
+                art X = P; wf y = z;
+                add_body(C, X);
                 to_J<T>(J, X, y);
                 bad |= eliminate<T, false>(X, y, nullptr, g);
-                if (oPP) {
-                    art Y = X;
-                    dm Rj = R;          // Ground rotation of the J axes
-                    if constexpr (T == UNIVERSAL) {
-                        const dm Ry = {{J.c1, 0, J.s1, 0, 1, 0, -J.s1, 0, J.c1}};
-                        Rj = chain::mulABt(R, Ry);
-                    } else if constexpr (T == FREE) Rj = chain::mulABt(R, J.R);
-                    put(oPP.from(21*b), Y, Rj, J.fromB(c.Bo(C)));
-                }
                 R = in_R<T, IDF>(C, J, R);
                 to_F<T, false>(J, X, y);
                 to_parent<T, IDF, false>(C, X, y, arm<T, IDF>(C, J));
@@ -443,21 +509,26 @@ __global__ void __launch_bounds__(64) k_cop(OpArgs a) {
                 constexpr int T = decltype(t)::t;
                 const cdptr C = c.C(b);
                 const Jnt<T> J = c.template joint_of<T>(x);
-                m += C[JC_M]; mc = mc + d3{C[JC_C], C[JC_C + 1], C[JC_C + 2]};
-#pragma unroll
-                for (int k = 0; k < 6; ++k) I.a[k] += C[JC_I + k];
                 {
+                    // about Bo: the children's share moved there, and the body's own
                     const d3 k0 = mc; const sym I0 = I;
+                    const auto own = c.own(b);
                     move(-c.Bo(C));
-                    const double oo = 1.0 / m;
+                    mc = mc + own.mc;
+#pragma unroll
+                    for (int k = 0; k < 6; ++k) I.a[k] += own.I.a[k];
+                    const double mt = m + own.m, oo = 1.0/mt;
                     const d3 pc = mul(R, oo*mc);
                     const sym Ig = rot(R, I);
                     const Pk o = ob.from(10*b);
-                    o(0) = m; o(1) = pc.x; o(2) = pc.y; o(3) = pc.z;
+                    o(0) = mt; o(1) = pc.x; o(2) = pc.y; o(3) = pc.z;
 #pragma unroll
                     for (int k = 0; k < 6; ++k) o(4 + k) = oo*Ig.a[k];
                     mc = k0; I = I0;
                 }
+                m += C[JC_M]; mc = mc + d3{C[JC_C], C[JC_C + 1], C[JC_C + 2]};
+#pragma unroll
+                for (int k = 0; k < 6; ++k) I.a[k] += C[JC_I + k];
                 R = in_R<T, IDF>(C, J, R);
                 const dm Rj = joint_rot<T>(J);
                 mc = fromF<IDF>(C, mul(Rj, mc)); I = rot(Rj, I);

@@ -1,6 +1,7 @@
 """Badly scaled models and states, each quantity on its own scale: a light fast
 distal link; a fast balanced wheel at the end of slow arms; angles next to
-the zeros of their cosine; a branch that is not a number beside one that is.
+the zeros of their cosine; a branch that is not a number beside one that is;
+a light last body whose joint lies far from it.
 
 Tolerances.  A recursion that forms every body's own values from its parent's
 is off by a few roundings of the quantity's own terms: with chains of three
@@ -223,3 +224,28 @@ def test_branch_beside_one_that_is_not_a_number():
     u = [np.array([0.1, 0.2]), np.zeros(1), np.array([0.1, 0.2])]
     ud = batch.split_u(batch.realizeAcceleration(batch.pack(q), batch.pack(u))[0])
     assert ud[0][0] == ud[2][0] and np.isnan(ud[0][1])
+
+
+@pytest.mark.parametrize("last", [M.PIN, M.UNIVERSAL, M.BALL, M.SLIDER])
+def test_leaf_inertias(last):
+    """Body frames at the mass center, joints 3 away, inertias of radius 0.001:
+    composite and articulated inertias about the body origins, the last body's
+    inertia blocks on their own size (what the joint's distance would add is 1e7
+    times as large)."""
+    from simbody_amd.matter import MatterBatch
+    spec = _planar([M.BALL, M.PIN, last], [1.0, 1.0, 1.0])
+    spec.com_B[:] = 0.0
+    spec.inertia_B[:] = 1e-6 * np.array([2.0, 3.0, 4.0, 0.1, 0.2, 0.3])
+    spec.X_BM[:, 9:] = [0.0, 3.0, 0.0]
+    q = np.concatenate([[0.5, 0.5, -0.5, 0.5], [0.3], [0.8, 0.0, 0.6, 0.0] if last == M.BALL else [0.7, -0.4][:M.NQ[last]]])
+    batch = MatterBatch([spec], n_instances=2)
+    Q = batch.pack([q, q])
+    P, PP = (np.reshape(batch.split_b(x, 21)[1], (-1, 21)) for x in batch.realizeArticulatedBodyInertias(Q))
+    C = np.reshape(batch.split_b(batch.calcCompositeBodyInertias(Q), 10)[1], (-1, 10))
+    o = OracleModel(spec)
+    oP, oPP = o.abi(q, spec.dofs())[:2]
+    oC = o.composite_inertias(q)
+    for got, ref in ((P[1:], oP), (PP[1:], oPP), (C[1:], oC[1:])):
+        assert np.abs(got - ref).max() < 1e-12 * np.abs(ref).max()
+    for got, ref in ((P[3, 6:12], oP[2, 6:12]), (PP[3, 6:12], oPP[2, 6:12]), (C[3, 4:], oC[3, 4:])):
+        assert np.abs(got - ref).max() < 1e-13 * np.abs(ref).max(), (got, ref)
