@@ -375,8 +375,10 @@ __global__ void __launch_bounds__(64) k_cop(OpArgs a) {
                 }
                 if constexpr (OP == OP_JAC || OP == OP_BACC) c.put_body(ob.from(6*b), C, R, A, VEL ? &w : nullptr);
                 if constexpr (OP == OP_KIN) {
-                    const wf h = rigid_force<false>(C, A, w);
-                    ke += 0.5 * (dot(A.w, h.w) + dot(A.v, h.v));
+                    // (about Bo, as the inertias below)
+                    const auto o = c.own(b);
+                    const d3 vb = A.v + cross(A.w, c.Bo(C));
+                    ke += 0.5 * (dot(A.w, mulsym(o.I, A.w) + cross(o.mc, vb)) + dot(vb, o.m*vb + cross(A.w, o.mc)));
                     const d3 cm = {C[JC_C], C[JC_C + 1], C[JC_C + 2]};
                     pe -= dot(grav, C[JC_M]*p + mul(R, cm));
                     if (ob) {

@@ -1,7 +1,8 @@
 """Badly scaled models and states, each quantity on its own scale: a light fast
 distal link; a fast balanced wheel at the end of slow arms; angles next to
 the zeros of their cosine; a branch that is not a number beside one that is;
-a light last body whose joint lies far from it.
+a small last body whose joint lies far from it; a small body that turns
+about itself.
 
 Tolerances.  A recursion that forms every body's own values from its parent's
 is off by a few roundings of the quantity's own terms: with chains of three
@@ -249,3 +250,21 @@ def test_leaf_inertias(last):
         assert np.abs(got - ref).max() < 1e-12 * np.abs(ref).max()
     for got, ref in ((P[3, 6:12], oP[2, 6:12]), (PP[3, 6:12], oPP[2, 6:12]), (C[3, 4:], oC[3, 4:])):
         assert np.abs(got - ref).max() < 1e-13 * np.abs(ref).max(), (got, ref)
+
+
+def test_kinetic_energy_of_a_spinning_leaf():
+    """A body of radius 0.001 that turns about its own mass center, the body
+    origin, while its Free joint's frame, 3 away, moves: the energy is that of
+    the turning alone, 1e-7 of what the joint frame's motion would suggest."""
+    from simbody_amd.matter import MatterBatch
+    spec = _planar([M.FREE], [1.0])
+    spec.com_B[:] = 0.0
+    spec.inertia_B[:] = 1e-6 * np.array([2.0, 3.0, 4.0, 0.1, 0.2, 0.3])
+    spec.X_BM[:, 9:] = [0.0, 3.0, 0.0]
+    batch = MatterBatch([spec], n_instances=2)
+    q = np.array([1.0, 0, 0, 0, 0.1, 0.2, 0.3])
+    w = np.array([0.75, -1.25, 0.5])
+    u = np.concatenate([w, np.cross(w, [0.0, 3.0, 0.0])])
+    E = batch.realizeKinematics(batch.pack([q, q]), batch.pack([u, u]))[3].cpu().numpy()
+    I = 1e-6 * np.array([[2.0, 0.1, 0.2], [0.1, 3.0, 0.3], [0.2, 0.3, 4.0]])
+    assert abs(E[2] - 0.5 * w @ I @ w) < 1e-13 * E[2]
