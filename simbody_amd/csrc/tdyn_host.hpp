@@ -4,8 +4,8 @@
 #include "../../include/tdyn.h"
 #include "tdyn_internal.hpp"
 
+#include <algorithm>
 #include <thread>
-#include <system_error>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -235,16 +235,16 @@ template <class Fn> void in_pieces(int n, int64_t work, Fn&& fn) {
     auto at = [&](int p) { return (int)((int64_t)n * p / m); };
     std::thread th[8];
     bool done[8] = {};
-    for (int p = 1; p < m; ++p) {
-        try {
-            th[p] = std::thread([&, p] {
-                try { fn(at(p), at(p + 1)); done[p] = true; } catch (...) {}
-            });
-        } catch (const std::system_error&) {}
-    }
     struct Join { std::thread* th; ~Join() { for (int p = 1; p < 8; ++p) if (th[p].joinable()) th[p].join(); } };
     {
         const Join join{th};
+        for (int p = 1; p < m; ++p) {
+            try {
+                th[p] = std::thread([&, p] {
+                    try { fn(at(p), at(p + 1)); done[p] = true; } catch (...) {}
+                });
+            } catch (...) { break; }        // (no thread, or no memory for one)
+        }
         fn(0, at(1));
     }
     for (int p = 1; p < m; ++p) if (!done[p]) fn(at(p), at(p + 1));
