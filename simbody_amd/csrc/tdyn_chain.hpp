@@ -76,8 +76,8 @@ struct PrmL {
 // A model whose frames are all identity rotations at the joints (R_PF = I,
 // p_PF = 0, R_MB = I; X_BM may translate), Simbody's noR_PF/noX_MB node
 // specializations: the products with those frames are skipped.  They are
-// exact in floating point (x*1 + y*0 + z*0 = x), so results are bitwise
-// those of the general form.
+// exact in floating point (x*1 + y*0 + z*0 = x); the builds still round
+// differently where the compiler fuses what is left of them.
 template <class PA> struct IdF {
     PA p;
     __device__ __forceinline__ IdF() = default;

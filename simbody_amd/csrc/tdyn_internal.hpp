@@ -212,10 +212,11 @@ hipError_t launch_op(OpKind k, const OpArgs& a, hipStream_t s);
 // The operator on a chain batch in joint frames (false: not one of these).
 bool launch_op_joint(OpKind k, const OpArgs& a, hipStream_t s);
 
-// Kinds of FP64 serving slots, by the request itself: identity rotations
-// between its joints, body forces that are not all zero.  Each has its own
-// build of the rollout.
-enum { SK_IDF = 1, SK_FORCES = 2, SK_N = 4 };
+// Kinds of serving slots, by the request itself: identity rotations between its
+// joints (mixed path: identity joint frames), and in FP64 body forces that are
+// not all zero.  Each has its own build of the rollout.  The mixed path keeps
+// the kind in body 1's PRM_KIND.
+enum { SK_IDF = 1, SK_FORCES = 2, SK_N = 4, PRM_KIND = PRM_PITCH };
 
 struct RkmArgs {
     DevTables T;
@@ -249,7 +250,7 @@ struct RkmArgs {
                              // or is a BendStretch
     const double* prm_lane;  // chain evaluator with one model per lane (serving slots), nullable:
                              // row k of lane l at prm_lane[k*L + l], nb*PRM_STRIDE model rows then gravity (3)
-    int kinds;               // FP64 serving slots: a bit for each kind (SK_*) that some slot has
+    int kinds;               // serving slots: a bit for each kind (SK_*) that some slot has
     int vec_aos;             // 1: vectors lane-contiguous (entry k of lane l at ((v*L + l)*ny_max + k)) and
                              // the streaming tree evaluator (batches of different trees)
     int stream_dmax;         // streaming tree evaluator: deepest body of any tree
@@ -347,15 +348,16 @@ int tree_group_resident_waves();
 hipError_t launch_chain_fp64_batch(const RkmArgs& a, hipStream_t s, bool f0_only);
 hipError_t launch_chain_fp64_lane(const RkmArgs& a, hipStream_t s);   // serving slots of the kinds a.kinds
 hipError_t launch_chain_mixed_batch(const RkmArgs& a, hipStream_t s, bool f0_only);
-hipError_t launch_chain_mixed_lane(const RkmArgs& a, hipStream_t s, bool f0_only);
+hipError_t launch_chain_mixed_lane(const RkmArgs& a, hipStream_t s);
 // precision 2, 3: FP64 arithmetic, single-precision G (and, 3, trig cache) rows
 hipError_t launch_chain_split_batch(const RkmArgs& a, hipStream_t s, bool f0_only);
 inline hipError_t launch_chain_variant(const RkmArgs& a, hipStream_t s, bool f0_only) {
     if (a.precision >= 2 && !a.prm_lane) return launch_chain_split_batch(a, s, f0_only);
-    if (a.precision == 1)
-        return a.prm_lane ? launch_chain_mixed_lane(a, s, f0_only) : launch_chain_mixed_batch(a, s, f0_only);
-    if (a.prm_lane) return f0_only ? hipErrorInvalidValue : launch_chain_fp64_lane(a, s);
-    return launch_chain_fp64_batch(a, s, f0_only);
+    if (a.prm_lane) {
+        if (f0_only) return hipErrorInvalidValue;
+        return a.precision == 1 ? launch_chain_mixed_lane(a, s) : launch_chain_fp64_lane(a, s);
+    }
+    return a.precision == 1 ? launch_chain_mixed_batch(a, s, f0_only) : launch_chain_fp64_batch(a, s, f0_only);
 }
 hipError_t launch_rkm(const RkmArgs& a, hipStream_t s);
 // Level-parallel tree evaluator (wavefront plan a.plan): rollout steps, or

@@ -36,6 +36,8 @@ __global__ void __launch_bounds__(64) k_rkm_chain(RkmArgs a) {
     const int lane = blockIdx.x * blockDim.x + threadIdx.x;
     if (lane >= a.n_inst) return;
     if (a.status[lane] != 0) return;
+    if constexpr (PrmTraits<PA>::lane)
+        if (a.prm_lane[(size_t)PRM_KIND * a.L + lane] != (PrmTraits<PA>::idf ? SK_IDF : 0)) return;
     const ChainEval<PA, K, GS, TS> ev(a, lane, 0);
     const int4 ta = ldi4(a.T.tree_a, 0);
     const int nb = ta.x, nq = ta.y, nu = ta.z, ny = nq + nu;

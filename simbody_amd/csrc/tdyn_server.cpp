@@ -39,8 +39,7 @@ struct tdyn_server {
     Pinned<int> slot_host, outi_host, status_host;
     std::vector<int> free_list;
     std::vector<char> occupied;
-    bool idf = false;      // every model admitted so far has identity joint frames (mixed path)
-    std::vector<signed char> kind;      // FP64: SK_* of each occupied slot
+    std::vector<signed char> kind;      // SK_* of each occupied slot
     int n_kind[SK_N] = {};              // and how many of each there are
     ~tdyn_server() { if (B) tdyn_batch_destroy(B); }
     int rec_stride() const { return nb * PRM_STRIDE + 3 + nq + nu + 1 + 6 * (nb + 1); }
@@ -48,7 +47,6 @@ struct tdyn_server {
         RkmArgs a = B->rk();
         a.chain = 1;
         a.prm_lane = prm_lane.p;
-        a.idf = idf ? 1 : 0;
         for (int k = 0; k < SK_N; ++k) a.kinds |= n_kind[k] > 0 ? 1 << k : 0;
         return a;
     }
@@ -118,7 +116,6 @@ int tdyn_server_create(const tdyn_tree_desc* topology, const tdyn_integrator_cfg
         delete S;
         return hipfail(e, "tdyn_server_create: device allocation");
     }
-    S->idf = identity_frames(*topology);
     S->free_list.resize(n);
     for (size_t i = 0; i < n; ++i) S->free_list[i] = (int)(n - 1 - i);    // pop_back gives slot 0 first
     S->occupied.assign(n, 0);
@@ -172,12 +169,9 @@ int tdyn_server_admit(tdyn_server* sv, int n, const tdyn_tree_desc* trees, const
             }
     });
     if (bad.load() < n) return check(bad.load());
-    // a model with general frames switches the server to the general kernel for good
-    for (int i = 0; i < std::min<int>(n, (int)sv->free_list.size()); ++i)
-        if (sv->idf && !identity_frames(trees[i])) sv->idf = false;
     const int k = std::min<int>(n, (int)sv->free_list.size());
     if (k == 0) return TDYN_OK;
-    const int stride = sv->rec_stride();
+    const int stride = sv->rec_stride(), row = sv->B->precision == 0 ? (int)JC_KIND : (int)PRM_KIND;
     HIPCHK(sv->rec_host.reserve((size_t)k * stride));
     HIPCHK(sv->slot_host.reserve(k));
     if (sv->rec_dev.n < (size_t)k * stride) HIPCHK(sv->rec_dev.alloc((size_t)std::max(k, 64) * stride));
@@ -203,14 +197,15 @@ int tdyn_server_admit(tdyn_server* sv, int n, const tdyn_tree_desc* trees, const
             for (int j = 0; j < 6 * (nb + 1); ++j) x[j] = fapp ? fapp[(size_t)i * 6 * (nb + 1) + j] : 0.0;
             // (Ground's force is not applied)
             const bool forces = std::any_of(x + 6, x + 6 * (nb + 1), [](double f) { return f != 0.0; });
-            if (sv->B->precision == 0) r[JC_KIND] = (identity_joints(r, nb) ? SK_IDF : 0) + (forces ? SK_FORCES : 0);
+            r[row] = row == PRM_KIND ? identity_frames(d) ? SK_IDF : 0
+                                     : (identity_joints(r, nb) ? SK_IDF : 0) + (forces ? SK_FORCES : 0);
         }
     });
     for (int i = 0; i < k; ++i) {
         const int slot = sv->free_list.back();
         sv->free_list.pop_back();
         sv->occupied[slot] = 1;
-        sv->kind[slot] = sv->B->precision == 0 ? (signed char)sv->rec_host.p[(size_t)i * stride + JC_KIND] : 0;
+        sv->kind[slot] = (signed char)sv->rec_host.p[(size_t)i * stride + row];
         ++sv->n_kind[(int)sv->kind[slot]];
         sv->slot_host.p[i] = slot;
         slots[i] = slot;

@@ -1,7 +1,8 @@
 """A request's result does not depend on its neighbours' options: with body
 forces or without (or with all of them zero), with identity joint frames or
 general ones, served alone, in a mixed burst, or in flight when a request of
-the other kind is admitted: equal to the bit, in both servers."""
+the other kind is admitted: equal to the bit, in the tree server and in the
+chain server at both precisions."""
 import numpy as np
 import pytest
 
@@ -34,10 +35,10 @@ def _requests(tree_server, n=12):
     return specs, [y[0] for y in ys], [y[1] for y in ys], np.linspace(0.2, 0.4, n), F
 
 
-def _server(tree_server, specs):
+def _server(tree_server, specs, precision):
     from simbody_amd.matter import RungeKuttaMerson
     from simbody_amd.serving import Server, TreeServer
-    integ = RungeKuttaMerson(accuracy=1e-5)
+    integ = RungeKuttaMerson(accuracy=1e-5, precision=precision)
     return TreeServer(integ, 1 << 28, max_slots=64) if tree_server else Server(specs[0], integ, 1 << 28, max_slots=64)
 
 
@@ -64,16 +65,16 @@ def _finish(sv, tree_server, at, out):
     raise AssertionError("requests did not finish")
 
 
-@pytest.mark.parametrize("tree_server", [False, True])
-def test_alone_and_beside_other_kinds(tree_server):
+@pytest.mark.parametrize("tree_server,precision", [(False, 0), (False, 1), (True, 0)])
+def test_alone_and_beside_other_kinds(tree_server, precision):
     req = _requests(tree_server)
     n = len(req[0])
     alone = {}
     for i in range(n):
-        sv = _server(tree_server, req[0])
+        sv = _server(tree_server, req[0], precision)
         alone.update(_finish(sv, tree_server, _admit(sv, tree_server, req, [i], bool(np.any(req[4][i]))), {}))
     # one burst of all kinds
-    sv = _server(tree_server, req[0])
+    sv = _server(tree_server, req[0], precision)
     burst = _finish(sv, tree_server, _admit(sv, tree_server, req, list(range(n)), True), {})
     # one after the other, each in flight when the next kind comes, on a server that has served all kinds
     late, at = {}, {}
