@@ -4,8 +4,7 @@
 namespace tdyn {
 
 hipError_t launch_chain_mixed_batch(const RkmArgs& a, hipStream_t s, bool f0_only) {
-    // the derivative alone (f0_only) is the general form's bit for bit, so
-    // identity frames need no separate build there
+    // (the derivative alone has one build, the general one: it agrees to rounding)
     if (a.idf && !f0_only) return launch_chain_t<chain::IdF<cdptr>, float>(a, s, false);
     return launch_chain_t<cdptr, float>(a, s, f0_only);
 }

@@ -2420,8 +2420,6 @@ __global__ void __launch_bounds__(64) k_tree_f0(RkmArgs a) {
 hipError_t launch_rollout_f0(const RkmArgs& a, hipStream_t s) {
     if (a.n_inst <= 0) return hipSuccess;
     const dim3 grd((a.n_inst + 63)/64), blk(64);
-    // the derivative is the general form's bit for bit, so identity frames
-    // need no separate build here
     if (a.chain) return launch_chain_variant(a, s, true);
     if (a.grp) return launch_tree_group(a, s, true);
     if (a.vec_aos) k_tree_f0<TreeStreamEval, false><<<grd, blk, 0, s>>>(a);

@@ -2,17 +2,24 @@
 // (tdyn_joint.hpp): one lane per instance, the sweep state in registers.
 //
 // The record-based sweeps (k_op) write and read 0.7-1.6 kB per body between
-// sweeps.  Here a sweep keeps 6 to 12 doubles per body for the next one (G and
-// DI*eps, the body's angular velocity, or the force on it), the joint angles' sines are formed again,
-// and rotations are recovered on the way back along the chain; the rest of the
-// traffic is the arguments and the results themselves.
+// sweeps.  Here a sweep keeps 3 to 12 doubles per body for the next one (the
+// body's angular velocity, G and DI*eps, or the force on it), the joint angles'
+// sines are formed again, and rotations are recovered on the way back along the
+// chain; the rest of the traffic is the arguments and the results themselves.
 //
 // Velocities and accelerations are not recovered from the tip's: a slow body's
 // would carry the rounding of a fast outer one's.  So each body's force is
 // formed on the way out, from the body's own acceleration, and kept.  (M v,
 // the residual and the reactions with everything recovered: base torque of a
 // two-link chain off by 7e-10 where the tip is 1e-8 of the link's mass and as
-// much faster.  65,536 x 32 inverse dynamics: 180 us so, 203 as it is.)
+// much faster.  65,536 x 32 inverse dynamics: 180 us so, 202 as it is; M v 116
+// and 178; realizeAcceleration 290 and 303.)
+//
+// What bounds it: at 65,536 chains the traffic (realizeAcceleration 1.26 GB at
+// 4.2 TB/s, inverse dynamics 0.83 GB at 4.1, of the 4.9 a plain copy reaches;
+// packed arguments at a lane stride are fetched several times), at a few chains
+// the issue and the loads of single wavefronts (52 % of the cycles issuing, 45 %
+// waiting).
 #include "tdyn_joint.hpp"
 
 namespace tdyn {

@@ -14,16 +14,20 @@
 //
 // The angular velocities are kept for the sweep back too (three doubles per
 // body, in the rows of its G).  Recovered from the tip's by subtraction they
-// moved 15 % fewer bytes (65,536 x 32: 11.2 ms for 16 steps, 12.6 as it is),
+// moved 12 % fewer bytes (65,536 x 32: 11.2 ms for 16 steps, 12.6 as it is),
 // but a slow body's carried the rounding of a fast outer one's: udot of two
-// arms with a balanced wheel at 1e7 rad/s was off by 5e-11.
+// arms with a balanced wheel at 1e7 rad/s was off by 5e-11.  (Those of every
+// second body only, the others formed from their parents': 5 % faster at this
+// size, 4 to 5 % slower for one chain and for 4,001.)
 //
 // What bounds it.  65,536 chains of 32 bodies are one wavefront per SIMD; a
-// step moves 57 kB per instance between the sweeps (half of it G and DI*eps)
-// at BW TB/s, near what a plain copy reaches, and issues half as many vector
-// instructions as the Ground-frame sweeps did: 0.79 ms per step against
-// 1.43 ms.  A few chains are bound by the latency of one lane's serial sweeps
-// (one 10-link pendulum: 1.6 against 3.4 ms for 0.1 s at accuracy 1e-8).
+// step moves 56 kB per instance between the sweeps (half of it G and DI*eps)
+// at 4.7 TB/s, near the 4.9 that a plain copy reaches, and issues half as many
+// vector instructions as the Ground-frame sweeps did: 0.77 ms per step against
+// 1.43 ms.  A few chains are bound by the instruction issue of single
+// wavefronts: 430 vector instructions a body and sweep, 66 % of the cycles
+// issuing and 29 % waiting (one 10-link pendulum: 1.3 against 2.6 ms for 0.1 s
+// at accuracy 1e-8).
 #pragma once
 #include "tdyn_joint.hpp"
 #include "tdyn_rkm_chain.hpp"

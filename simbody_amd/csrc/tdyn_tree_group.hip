@@ -543,7 +543,8 @@ __global__ void k_zero_int(int* p, int n) {
 } // namespace
 
 // a.idf: every R_MF is the identity and the products with it are skipped (the
-// results are bitwise those of the general form).  a.ext: some mobilizer is
+// same results but for the last bits, where the compiler fuses what is left).
+// a.ext: some mobilizer is
 // reversed, uses Euler angles or is a BendStretch or Bushing, or some bodies
 // have known udot: the Ground-frame evaluator.
 template <class EV> static void launch_plan(const RkmArgs& a, hipStream_t s, bool f0_only) {

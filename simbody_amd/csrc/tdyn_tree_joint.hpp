@@ -6,10 +6,11 @@
 // on the angular velocity (and the rotation where body forces are given) in
 // place of a pose and a velocity.
 //
-// What bounds it: the chain of steps, each a serial run of about 1,500
-// instructions of one wavefront per SIMD, and the memory behind it (16,384
-// trees: 180 MB of records, constants and vectors in use at a time, 3 TB/s
-// between L2 and what lies behind it).  Hence:
+// What bounds it: the memory behind the records (16,384 trees: 180 MB of
+// records, constants and vectors in use at a time; a rollout moves 21 GB at 4.2
+// TB/s, realizeAcceleration 1.43 GB at 3.9, of the 4.9 a plain copy reaches),
+// and in smaller batches the chain of steps, each a serial run of about 1,500
+// instructions of one wavefront per SIMD.  Hence:
 // - steps of up to G positions of the breadth-first order, cut where a
 //   position's parent (child) is in the step, not at the levels: 11.1 steps
 //   for a mean tree of 8 to 128 bodies and 8 lanes where the levels make 12.7;
@@ -19,10 +20,10 @@
 // - one sweep inward and one outward per derivative of a rollout: the outward
 //   sweep forms the next stage's state and passes on its angular velocities.
 // 16,384 trees of 8 to 128 bodies with forces, 16 lanes each: realize
-// acceleration 371 us (one lane per tree: 3,230); a rollout derivative 490 us,
-// where the Ground-frame evaluator of three sweeps took 1,000.  With 8 lanes
-// a rollout took 10.7 ms for 8.4 with 16, as twice the records are in use,
-// and with 32 lanes 10.5.
+// acceleration 371 us (one lane per tree: 3,230); a rollout to 0.02 s 5.9 ms
+// (Ground frames, three sweeps a derivative: 11.8).  With 4 / 8 / 32 lanes the
+// rollout takes 13.8 / 7.9 / 7.1 ms: with fewer, more records are in use at a
+// time, with more, most lanes idle.
 #pragma once
 #include "tdyn_joint.hpp"
 #include "tdyn_joint_const.hpp"
